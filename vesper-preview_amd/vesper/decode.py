@@ -27,6 +27,7 @@ from torch import Tensor
 
 from vesper.attention import rotary_inv_freq
 from vesper.contracts import ContractError, Dims, check_shape
+from vesper.kernels.carry import residual_rows_where
 from vesper.kernels.delta_scan import delta_scan_step_fused, delta_scan_step_keys
 from vesper.kernels.norm import decode_projection
 from vesper.kernels.ring_attn import RingKVCache, ring_attention
@@ -125,7 +126,8 @@ def decode_step(column: LoopedColumn, depth: int, values: Sequence[Tensor],
             a, _ = ring_attention(aq, ak, av.view(b, 1, hkv, dk), position, ring, inplace=True, check_positions=False,
                                   workspace=workspace)
             pending = a.reshape(b, hd)
-        x = (xs + pending).view(b, 1, d)  # float32 (promoted in the add)
+        x = torch.empty(b, 1, d, device=xs.device)
+        residual_rows_where(xs.view(b, 1, d), pending.view(b, 1, d), x, None)  # float32 (promoted in the add)
     return [x, *flat]
 
 
