@@ -315,3 +315,23 @@ def test_decode_config_256_steps_delta_and_ring_against_the_chunked_oracles():
     # the ring now holds positions 256..767: slots 0..255 rewritten with the new tokens
     assert torch.equal(ring.pos[:, :steps].cpu(), torch.arange(w, w + steps).expand(b, steps))
     assert torch.equal(ring.k[:, :steps].cpu(), ak) and torch.equal(ring.v[:, steps:].cpu(), rv[:, steps:])
+
+
+@pytest.mark.parametrize(("h", "hkv", "dk"), [(1, 1, 8), (3, 1, 16), (8, 8, 32), (8, 4, 64), (12, 4, 64), (8, 2, 64),
+                                              (8, 1, 64), (6, 1, 128), (8, 1, 256), (7, 1, 24)])
+@pytest.mark.parametrize("w", [1, 255, 257, 1030])
+def test_the_merge_over_key_groups_at_the_edges_of_a_batch(h, hkv, dk, w):
+    """Every lane layout of a key row (one lane to 32) and every group size, over windows of one slot,
+    one off a batch of keys and several batches with a remainder. The output is a bf16 rounding
+    (2^-9 relative) of a float32 sum of at most 1031 terms (2^-24 each, times exponents' few ulp)."""
+    from vesper.kernels.ring_attn import RingKVCache, ring_attention
+
+    b = 2
+    rk, rv, rpos, valid, p = _random_ring(b, w, hkv, dk, seed=w + dk + h)
+    g = torch.Generator().manual_seed(9)
+    q = torch.randn(b, 1, h, dk, generator=g).to(BF16)
+    k = torch.randn(b, 1, hkv, dk, generator=g).to(BF16)
+    v = torch.randn(b, 1, hkv, dk, generator=g).to(BF16)
+    want = oa.ring_attend(q.double(), k.double(), v.double(), p, rk.double(), rv.double(), rpos, valid, w)
+    o, _ = ring_attention(q.to(GPU), k.to(GPU), v.to(GPU), p.to(GPU), RingKVCache(*(t.to(GPU) for t in (rk, rv, rpos, valid)), w))
+    torch.testing.assert_close(o.double().cpu(), want, rtol=2**-8, atol=2**-14)

@@ -13,7 +13,7 @@
 // arithmetic, so the whole window of the head is in flight at once (W = 512 at D = 64 is one
 // batch). Each thread keeps, per query head, an online softmax over its own keys (running max,
 // sum and weighted values, base-2 exponent); the partial states merge across the key groups of a
-// wave with lane shuffles and across the waves through LDS, in a fixed order.
+// wave in registers and across the waves through LDS, in a fixed order.
 //
 // The write: a workgroup writes its own KV head's key and value into slot p % W after all of its
 // reads (no other workgroup reads that head). The slot's position and valid flag are shared by the
@@ -33,17 +33,19 @@ namespace {
 constexpr int kMaxGroup = 8;
 
 // The workgroup shape by GM, the query heads per KV head rounded up to a power of two (register
-// arrays are sized by it): groups of up to two query heads run 1024 threads with four keys each
-// (many waves per CU with few loads each stream the window faster than fewer waves with many loads:
-// 24.6 against 25.1 us per decode step with the ring read from HBM); wider groups run 256 threads
-// with eight keys each, so the per-head softmax states still fit in registers.
+// arrays are sized by it). Groups of up to two query heads run 1024 threads (many waves per CU with
+// few loads each stream the window faster than fewer waves with many loads: 24.6 against 25.1 us per
+// decode step with the ring read from HBM). Wider groups are bound by their arithmetic (about 0.8 us
+// a query head at W 512 D 64) and run 512 threads, the most whose registers hold their softmax states.
+// One row at W 512 D 64, four and eight query heads a KV head: 8.7 and 12.4 us, against 10.1 and
+// 13.7 with 256 threads of eight keys, 8.9 and 13.3 with 512 of eight, 9.6 and (spilling) 16.6 with 1024.
 template <typename T> struct Ring8 {
   typedef T V8 __attribute__((ext_vector_type(8)));
 };
 
 template <int GM> struct RingShape {
-  static constexpr int NT = GM <= 2 ? 1024 : 256;  // threads
-  static constexpr int KPT = GM <= 2 ? 4 : 8;      // keys per thread per batch
+  static constexpr int NT = GM <= 2 ? 1024 : 512;  // threads
+  static constexpr int KPT = 4;                    // keys per thread per batch
 };
 
 // Eight ring elements as the queries' type: the ring's own type is either the queries' (one 16-byte
@@ -73,6 +75,61 @@ __device__ __forceinline__ void store_ring8(R* p, const typename Ring8<T>::V8& x
     reinterpret_cast<float4*>(p)[0] = make_float4(to_f32(x[0]), to_f32(x[1]), to_f32(x[2]), to_f32(x[3]));
     reinterpret_cast<float4*>(p)[1] = make_float4(to_f32(x[4]), to_f32(x[5]), to_f32(x[6]), to_f32(x[7]));
   }
+}
+
+// The value of lane ^ OFF combined with the lane's own (OFF a power of two).
+template <int OFF, typename Op>
+__device__ __forceinline__ float xor_combine(float x, Op op) {
+  if constexpr (OFF == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else if constexpr (OFF == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else if constexpr (OFF == 8) {
+    return op(x, dpp_f32<0x128>(x));  // row_ror:8
+  } else {
+    return op(x, __shfl_xor(x, OFF));
+  }
+}
+// x combined over the wave's key groups: over the lanes that hold the same piece of a row (KL lanes a row)
+template <int KL, typename Op>
+__device__ __forceinline__ float key_group_reduce(float x, Op op) {
+  x = xor_combine<32>(x, op);
+  if constexpr (KL <= 16) x = xor_combine<16>(x, op);
+  if constexpr (KL <= 8) x = xor_combine<8>(x, op);
+  if constexpr (KL <= 4) x = xor_combine<4>(x, op);
+  if constexpr (KL <= 2) x = xor_combine<2>(x, op);
+  if constexpr (KL <= 1) x = xor_combine<1>(x, op);
+  return x;
+}
+// A lane's features after the sum over the key groups: eight, halved by each of at most three steps.
+template <int KL> constexpr int kFeaturesLeft = KL <= 8 ? 1 : (KL <= 16 ? 2 : 4);
+// f summed over the key groups: a lane keeps features e0 .. e0 + kFeaturesLeft - 1 of its piece in f[0 ..],
+// e0 from its lane bits 5, 4, 3 (feature bits 2, 1, 0).
+template <int KL>
+__device__ __forceinline__ void key_group_sum(float (&f)[8]) {
+  const auto add = [](float x, float y) { return x + y; };
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(f[e]), __float_as_uint(f[e + 4]), false, false);
+    f[e] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  if constexpr (KL <= 16) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(f[e]), __float_as_uint(f[e + 2]), false, false);
+      f[e] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+  }
+  if constexpr (KL <= 8) {
+    const bool up = (threadIdx.x & 8) != 0;
+    const float keep = up ? f[1] : f[0], send = up ? f[0] : f[1];
+    f[0] = keep + dpp_f32<0x128>(send);
+  }
+  if constexpr (KL <= 4) f[0] = xor_combine<4>(f[0], add);
+  if constexpr (KL <= 2) f[0] = xor_combine<2>(f[0], add);
+  if constexpr (KL <= 1) f[0] = xor_combine<1>(f[0], add);
 }
 
 template <typename T, typename R, int D, int GM, bool PAD>
@@ -249,27 +306,29 @@ __global__ __launch_bounds__(RingShape<GM>::NT) void ring_attn_kernel(
       fold(sc, vn, 1);
     }
 
-    // merge the partial softmax states: key groups of a wave, then the waves
+    // merge the partial softmax states: key groups of a wave, then the waves. Within a wave the states
+    // first take the wave's maximum; the sums then halve the features a lane holds at each step over
+    // the key groups (lane bit 5 takes feature bit 2, bit 4 bit 1, bit 3 bit 0), so eight features
+    // cost seven exchanges instead of 24, all in registers: one row at W 512 D 64, 6.15 -> 5.55 us
+    // with one query head a KV head, 11.4 -> 10.1 with four, 16.8 -> 13.7 with eight.
 #pragma unroll
     for (int gi = 0; gi < GM; ++gi) {
+      const float mw = key_group_reduce<KL>(m[gi], [](float x, float y) { return fmaxf(x, y); });
+      const float a = __builtin_amdgcn_exp2f(m[gi] - mw);
+      const float lw = key_group_reduce<KL>(l[gi] * a, [](float x, float y) { return x + y; });
+      float f[8];
 #pragma unroll
-      for (int off = KL; off < 64; off <<= 1) {
-        const float mo = __shfl_xor(m[gi], off);
-        const float lo = __shfl_xor(l[gi], off);
-        const float mn = fmaxf(m[gi], mo);
-        const float a = __builtin_amdgcn_exp2f(m[gi] - mn), c = __builtin_amdgcn_exp2f(mo - mn);
-        l[gi] = l[gi] * a + lo * c;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[gi][e] = acc[gi][e] * a + __shfl_xor(acc[gi][e], off) * c;
-        m[gi] = mn;
-      }
-      if (lane < KL) {
-        if (part == 0) {
-          smerge[wv][gi][0] = m[gi];
-          smerge[wv][gi][1] = l[gi];
+      for (int e = 0; e < 8; ++e) f[e] = acc[gi][e] * a;
+      key_group_sum<KL>(f);
+      constexpr int NF = kFeaturesLeft<KL>;
+      if ((lane & 7) < KL || KL > 8) {  // lanes past a narrow row's pieces hold copies
+        if (lane == 0) {
+          smerge[wv][gi][0] = mw;
+          smerge[wv][gi][1] = lw;
         }
+        const int e0 = (KL <= 32 && (lane & 32) ? 4 : 0) + (KL <= 16 && (lane & 16) ? 2 : 0) + (KL <= 8 && (lane & 8) ? 1 : 0);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) smerge[wv][gi][2 + 8 * part + e] = acc[gi][e];
+        for (int u = 0; u < NF; ++u) smerge[wv][gi][2 + 8 * part + e0 + u] = f[u];
       }
     }
     __syncthreads();
