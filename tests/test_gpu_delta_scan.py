@@ -262,6 +262,22 @@ def test_the_form_picked_by_shape_matches_the_oracle(b, n, h):
     assert relative_error(o, o_ref) < TOL and relative_error(s, s_ref) < TOL
 
 
+# 17 and 18 segments (an odd and an even number of folded maps), 31; either side of the line below
+# which the chains run (39 and 40 chunks of one head), each also one token off a whole chunk
+@pytest.mark.parametrize(("b", "n", "h"), [(1, 68 * 64 - 1, 1), (1, 72 * 64, 1), (1, 124 * 64 - 63, 1),
+                                           (1, 38 * 64 + 1, 1), (1, 39 * 64 + 1, 1), (5, 4033, 8)])
+def test_long_sequences_of_few_heads_by_shape_match_the_oracle_and_the_chains(b, n, h):
+    from vesper.kernels.delta_scan import delta_scan_fused
+
+    q, k, v, beta, h0 = _bf16_inputs(b, n, h, 64, seed=n)
+    o_ref, s_ref = _oracle(q, k, v, beta, h0)
+    o, s = _scan_form(2, delta_scan_fused, q, k, v, beta, h0)
+    oc, sc = _scan_form(0, delta_scan_fused, q, k, v, beta, h0)
+    # no further from float64 than the chains by more than a tenth (both round the state to bf16 a chunk)
+    assert relative_error(o, o_ref) < min(TOL, 1.1 * relative_error(oc, o_ref))
+    assert relative_error(s, s_ref) < min(TOL, 1.1 * relative_error(sc, s_ref))
+
+
 @pytest.mark.parametrize(("b", "n", "h"), SEGMENTED[:2])
 def test_the_segmented_scan_with_an_active_mask(b, n, h):
     from vesper.kernels.delta_scan import delta_scan_fused

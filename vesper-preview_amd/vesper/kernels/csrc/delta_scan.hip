@@ -1390,10 +1390,8 @@ void launch_chunked(const TIn* q, const TIn* k, const TIn* v, const TIn* beta, c
                      beta, tmat, active, carried.k, carried.v, carried.beta, T, H, total, strength.m, strength.alpha,
                      strength.logits);
   if constexpr (std::is_same<TIn, __bf16>::value && DK == 64) {
-    // by shape: the value-slice chains while they fit one workgroup a CU (B H D/16 <= kSegBlocks),
-    // where their four CUs a head outrun one whole-head workgroup a segment; the segments beyond
     const int form = scan_segments();
-    if (form == 1 || (form == 2 && B * H * (DK / 16) > kSegBlocks)) {
+    if (form == 1 || (form == 2 && seg_faster(B, H, T))) {
       launch_segments<CARRY>(q, k, v, s_in, s_out, o, tmat, active, carried, B, T, H, stream, hrec);
       return;
     }

@@ -10,12 +10,17 @@
 //
 //  * delta_seg_kernel<kSegMaps> runs every segment but the last once without outputs, carrying
 //    [X | M] through its chunks (M from I, X from zero; the first segment carries the true state
-//    from S0 instead and needs no M), and writes X and M (fp32, row-major [64][64]) to the
-//    workspace; its first segment also copies S0 there, so that the output pass may write the
-//    final state over S0 (s_out == s_in) while its first segment still reads the copy;
+//    from S0 instead and needs no M), and writes X (fp32, accumulator order) and M (bf16 A fragments
+//    of its high parts and of what they leave) to the workspace; its first segment also copies S0
+//    there, so that the output pass may write the final state over S0 (s_out == s_in) while its
+//    first segment still reads the copy;
 //  * delta_seg_kernel<kSegOutputs> starts segment s from H = X_0, folded through the maps of
-//    segments 1 .. s - 1 (H <- X_i + M_i H, three bf16 products per tile: hi*hi + hi*lo + lo*hi),
-//    then runs its chunks with the outputs; the last segment writes the final state.
+//    segments 1 .. s - 1 (H <- X_i + M_i H, three bf16 products per tile: hi*hi + hi*lo + lo*hi; each
+//    map in two 16-byte loads a fragment, the next one's in flight), then runs its chunks with the
+//    outputs; the last segment writes the final state. The last segments' fold is the sequential
+//    part of a long sequence: with the maps as fp32 matrices, loaded and split as they were applied,
+//    it took about 1.6 us a map, now 0.3 (scan of B1 T8191, 2 / 12 / 24 heads: 81.5 / 67.6 / 64.4 us
+//    -> 44.5 / 50.4 / 59.1).
 //
 // Waves of a workgroup (512 threads):
 //  * waves 0-3, the chain: wave j keeps value columns 16 j .. 16 j + 15 of the state in MFMA
@@ -62,6 +67,19 @@ inline SegShape seg_shape(int B, int H, int T) {
   return SegShape{(nc + len - 1) / len, len};
 }
 constexpr size_t kSegMapBytes = 2 * 64 * 64 * sizeof(float);  // X and M of one (b, h, segment)
+
+// Whether the segments outrun the value-slice chains. Past one chain workgroup a CU (four a head)
+// the chains queue, and the segments win. Below that, in tenths of a microsecond: a chain takes about
+// 6 a chunk; the two passes take about 110 more to start than it, 22 a chunk of a segment (8 the
+// maps, 14 the outputs) and 3 a map folded. Measured chains / segments, us: B H 12, T 2048 28.2 /
+// 30.2, T 4096 47.0 / 39.0, T 8191 83.3 / 50.4; B H 40, T 4096 54.5 / 52.0; B H 48, T 4096 55.2 /
+// 56.8, T 8191 92.9 / 88.2; B H 64, T 4096 60.1 / 65.6.
+inline bool seg_faster(int B, int H, int T) {
+  if ((long)B * H * 4 > kSegBlocks) return true;
+  const SegShape sh = seg_shape(B, H, T);
+  const int nc = (T + kChunk - 1) / kChunk;
+  return 6L * nc > 110 + 22L * sh.seglen + 3L * sh.nseg;
+}
 
 template <int MODE, bool CARRY>
 __global__ __launch_bounds__(512) void delta_seg_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k,
@@ -166,11 +184,28 @@ __global__ __launch_bounds__(512) void delta_seg_kernel(const __bf16* __restrict
           for (int r = 0; r < 4; ++r) head_s0[(16 * m + 4 * g + r) * DK + 16 * j + lq] = hreg[m][r];
       }
     } else if (OUT) {
+      // the maps of segments 1 .. sg - 1, the next one's loads in flight while this one is applied
+      struct Fold {
+        bf16x8 hi[4][KBF], lo[4][KBF];  // M's A fragments: row tile m, dk block kb
+        f32x4 x[4];
+      };
+      const float* seg_x = head_maps + (j * 4 * 64 + l) * 4;
+      const E* seg_m = reinterpret_cast<const E*>(head_maps + DK * DK) + 8 * l;
+      constexpr size_t kStep = kSegMapBytes / sizeof(float);
+      auto fetch = [&](Fold& f, int i) {
+        const float* X = seg_x + (size_t)i * kStep;
+        const E* M = seg_m + (size_t)i * kStep * 2;
 #pragma unroll
-      for (int m = 0; m < 4; ++m) hreg[m] = load_tile(head_maps, m);  // X_0 = the state after segment 0
-      for (int i = 1; i < sg; ++i) {
-        const float* X = head_maps + (size_t)i * (kSegMapBytes / sizeof(float));
-        const float* M = X + DK * DK;
+        for (int m = 0; m < 4; ++m) {
+#pragma unroll
+          for (int kb = 0; kb < KBF; ++kb) {
+            f.hi[m][kb] = *reinterpret_cast<const bf16x8*>(M + (m * KBF + kb) * FR);
+            f.lo[m][kb] = *reinterpret_cast<const bf16x8*>(M + (8 + m * KBF + kb) * FR);
+          }
+          f.x[m] = *reinterpret_cast<const f32x4*>(X + m * 256);
+        }
+      };
+      auto apply = [&](const Fold& f) {  // H <- X + M H
         bf16x8 hhi[KBF], hlo[KBF];
 #pragma unroll
         for (int kb = 0; kb < KBF; ++kb) {
@@ -182,29 +217,28 @@ __global__ __launch_bounds__(512) void delta_seg_kernel(const __bf16* __restrict
           }
         }
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          f32x4 acc = load_tile(X, m);
+        for (int m = 0; m < 4; ++m) hreg[m] = f.x[m];
 #pragma unroll
-          for (int kb = 0; kb < KBF; ++kb) {
-            // A fragment of M: row 16 m + lq, dk 32 kb + 4 g .. + 3 and 32 kb + 16 + 4 g .. + 3
-            const f32x4 lo4 = *reinterpret_cast<const f32x4*>(M + (16 * m + lq) * DK + 32 * kb + 4 * g);
-            const f32x4 hi4 = *reinterpret_cast<const f32x4*>(M + (16 * m + lq) * DK + 32 * kb + 16 + 4 * g);
-            bf16x8 ahi, alo;
+        for (int kb = 0; kb < KBF; ++kb) {  // four independent sums in turn
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              ahi[r] = (__bf16)lo4[r];
-              ahi[4 + r] = (__bf16)hi4[r];
-              alo[r] = (__bf16)(lo4[r] - (float)ahi[r]);
-              alo[4 + r] = (__bf16)(hi4[r] - (float)ahi[4 + r]);
-            }
-            acc = mfma_bf16(ahi, hhi[kb], acc);
-            acc = mfma_bf16(ahi, hlo[kb], acc);
-            acc = mfma_bf16(alo, hhi[kb], acc);
-          }
-          mreg[m] = acc;  // the folded state, moved to hreg once every tile has read the old one
+          for (int m = 0; m < 4; ++m) hreg[m] = mfma_bf16(f.hi[m][kb], hhi[kb], hreg[m]);
+#pragma unroll
+          for (int m = 0; m < 4; ++m) hreg[m] = mfma_bf16(f.hi[m][kb], hlo[kb], hreg[m]);
+#pragma unroll
+          for (int m = 0; m < 4; ++m) hreg[m] = mfma_bf16(f.lo[m][kb], hhi[kb], hreg[m]);
         }
+      };
 #pragma unroll
-        for (int m = 0; m < 4; ++m) hreg[m] = mreg[m];
+      for (int m = 0; m < 4; ++m) hreg[m] = *reinterpret_cast<const f32x4*>(seg_x + m * 256);  // X_0: the state after segment 0
+      Fold f0, f1;
+      if (sg > 1) fetch(f0, 1);
+      for (int i = 1; i < sg; i += 2) {
+        if (i + 1 < sg) fetch(f1, i + 1);
+        apply(f0);
+        if (i + 1 < sg) {
+          if (i + 2 < sg) fetch(f0, i + 2);
+          apply(f1);
+        }
       }
     } else {
 #pragma unroll
@@ -318,12 +352,27 @@ __global__ __launch_bounds__(512) void delta_seg_kernel(const __bf16* __restrict
         for (int m = 0; m < 4; ++m) store_tile(s_out + (size_t)bh * DK * DK, m, hreg[m]);
       }
     } else {
+      // X in accumulator order, and M as the fold multiplies it: bf16 A fragments of its high parts,
+      // then of what they leave
       float* X = maps + ((size_t)bh * nmap + sg) * (kSegMapBytes / sizeof(float));
 #pragma unroll
-      for (int m = 0; m < 4; ++m) store_tile(X, m, hreg[m]);
+      for (int m = 0; m < 4; ++m) {
+        const float nan = __builtin_nanf("");
+        *reinterpret_cast<f32x4*>(X + ((j * 4 + m) * 64 + l) * 4) = bad ? f32x4{nan, nan, nan, nan} : hreg[m];
+      }
       if (with_m) {
+        E* M = reinterpret_cast<E*>(X + DK * DK);
+        // element (16 m + 4 g + r, 16 j + lq) lies in fragment (m, j / 2), on the lane of row 4 g + r and
+        // column group lq / 4, as element 4 (j % 2) + lq % 4
+        E* at = M + (j >> 1) * FR + ((lq >> 2) * 16 + 4 * g) * 8 + 4 * (j & 1) + (lq & 3);
 #pragma unroll
-        for (int m = 0; m < 4; ++m) store_tile(X + DK * DK, m, mreg[m]);
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const __bf16 hi = (__bf16)mreg[m][r];
+            at[m * KBF * FR + r * 8] = hi;
+            at[(8 + m * KBF) * FR + r * 8] = (__bf16)(mreg[m][r] - (float)hi);
+          }
       }
     }
     return;
