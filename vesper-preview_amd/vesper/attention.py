@@ -93,7 +93,7 @@ def kv_cache_push(cache: KVCache, k: Tensor, v: Tensor, pos: Tensor) -> KVCache:
                   torch.empty(b, keep, hkv, dk, dtype=v.dtype, device=k.device),
                   torch.empty(b, keep, dtype=torch.long, device=k.device), w)
     ck, cv, cp, kk, vv, pp = (t.contiguous() for t in (cache.k, cache.v, cache.pos, k, v, pos))
-    with torch.cuda.device(k.device):
+    with _lib.on_device(k.device):
         _lib.call("vsp_kv_cache_push", ck.data_ptr(), cv.data_ptr(), cp.data_ptr(), kk.data_ptr(), vv.data_ptr(),
                   pp.data_ptr(), out.k.data_ptr(), out.v.data_ptr(), out.pos.data_ptr(), b, m, n, hkv, dk,
                   k.element_size(), w, _lib.stream_of(k.device))
@@ -146,7 +146,7 @@ def _launch_rotary(q: Tensor, k: Tensor | None, pos: Tensor, base: float) -> tup
     qo = torch.empty_like(qc)
     ko = None if kc is None else torch.empty_like(kc)
     pc = pos.contiguous()
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         _lib.call(f"vsp_rotary_qk_{_SUFFIX[q.dtype]}", qc.data_ptr(), _lib.ptr(kc), pc.data_ptr(),
                   _inv_freq(base, dk, q.device).data_ptr(), qo.data_ptr(), _lib.ptr(ko), b, n, h, hkv, dk,
                   _lib.stream_of(q.device))

@@ -23,21 +23,25 @@ def check_shape(name: str, tensor: torch.Tensor, spec: DimSpec, dims: Dims, dtyp
     Raises:
         ContractError: on a rank, dimension or dtype mismatch.
     """
-    shape = tuple(tensor.shape)
+    shape = tensor.shape
     if len(shape) != len(spec):
-        raise ContractError(f"{name}: expected rank {len(spec)} {spec}, got shape {shape}")
+        raise ContractError(f"{name}: expected rank {len(spec)} {spec}, got shape {tuple(shape)}")
+    bind = dims.setdefault
+    for want, got in zip(spec, shape):
+        if (want if want.__class__ is int else bind(want, got)) != got:
+            _refuse_shape(name, tuple(shape), spec, dims)
+    if dtype is not None and tensor.dtype != dtype:
+        raise ContractError(f"{name}: dtype must be {dtype}, got {tensor.dtype}")
+
+
+def _refuse_shape(name: str, shape: tuple[int, ...], spec: DimSpec, dims: Dims) -> None:
+    """Raises for the first axis of ``shape`` that does not meet ``spec`` under the bindings ``dims``."""
     for axis, (want, got) in enumerate(zip(spec, shape)):
         if isinstance(want, int):
             if got != want:
                 raise ContractError(f"{name}: axis {axis} must be {want}, got {got} (shape {shape})")
-            continue
-        bound = dims.get(want)
-        if bound is None:
-            dims[want] = got
-        elif bound != got:
-            raise ContractError(f"{name}: axis {axis} '{want}' is {got}, but '{want}' = {bound} elsewhere")
-    if dtype is not None and tensor.dtype != dtype:
-        raise ContractError(f"{name}: dtype must be {dtype}, got {tensor.dtype}")
+        elif dims[want] != got:
+            raise ContractError(f"{name}: axis {axis} '{want}' is {got}, but '{want}' = {dims[want]} elsewhere")
 
 
 def require(condition: torch.Tensor, message: str) -> None:

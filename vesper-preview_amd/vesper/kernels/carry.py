@@ -65,7 +65,7 @@ def copy_rows_where(items: Sequence[tuple[Tensor, Tensor, Tensor]]) -> None:
     dst_arr = (ctypes.c_void_p * count)(*[t.data_ptr() for t in dsts])
     flag_arr = (ctypes.c_void_p * count)(*[t.data_ptr() for t in flags])
     size_arr = (ctypes.c_size_t * count)(*sizes)
-    with torch.cuda.device(device):
+    with _lib.on_device(device):
         _lib.call("vsp_copy_rows_where", count, ctypes.cast(src_arr, ctypes.c_void_p),
                   ctypes.cast(dst_arr, ctypes.c_void_p), ctypes.cast(size_arr, ctypes.c_void_p),
                   ctypes.cast(flag_arr, ctypes.c_void_p), int(rows or 0), _lib.stream_of(device))
@@ -94,7 +94,7 @@ def halt_step(active: Tensor, exits: Tensor | None, n_iters: Tensor) -> tuple[Te
     e = None if exits is None else exits.contiguous()
     halts = torch.empty_like(a)
     nxt = torch.empty_like(a)
-    with torch.cuda.device(active.device):
+    with _lib.on_device(active.device):
         _lib.call("vsp_halt_step", a.data_ptr(), _lib.ptr(e), n_iters.data_ptr(), halts.data_ptr(), nxt.data_ptr(),
                   a.numel(), _lib.stream_of(active.device))
     return halts, nxt
@@ -130,6 +130,6 @@ def residual_rows_where(x1: Tensor, a: Tensor, x: Tensor, flags: Tensor | None) 
             raise ContractError(f"{name} must be 16-byte aligned")
     fl = None if flags is None else flags.contiguous().view(torch.uint8)
     b, n, d = x1.shape
-    with torch.cuda.device(x1.device):
+    with _lib.on_device(x1.device):
         _lib.call("vsp_residual_rows_where", x1c.data_ptr(), ac.data_ptr(), x.data_ptr(), _lib.ptr(fl), b * n, d,
                   _lib.stream_of(x1.device))

@@ -117,7 +117,7 @@ def _scan(entry: str, q: Tensor, k: Tensor, v: Tensor, beta: Tensor, state: Tens
     lib = _lib.library()
     ws_bytes = int(lib.vsp_delta_scan_workspace_bytes(b, n, h, dk, int(fp32)))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         if records is not None:  # the bf16 forward that also keeps the chunks' starting states
             _lib.call("vsp_delta_scan_record_bf16", q.data_ptr(), k.data_ptr(), v.data_ptr(), beta.data_ptr(),
                       state.data_ptr(), o.data_ptr(), s_out.data_ptr(), _lib.ptr(ws), ws_bytes, _lib.ptr(mask),
@@ -183,7 +183,7 @@ class _DeltaScan(torch.autograd.Function):
         ws_bytes = int(lib.vsp_delta_scan_backward_workspace_bytes(b, n, h, dk))
         ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q.device)
         entry = "vsp_delta_scan_backward_f32" if ctx.fp32 else "vsp_delta_scan_backward_bf16"
-        with torch.cuda.device(q.device):
+        with _lib.on_device(q.device):
             if records is not None:
                 _lib.call("vsp_delta_scan_backward_recorded_bf16", q.data_ptr(), k.data_ptr(), v.data_ptr(),
                           beta.data_ptr(), state.data_ptr(), go.data_ptr(), _lib.ptr(gs), _lib.ptr(mask),
@@ -319,7 +319,7 @@ def delta_scan_step_fused(q: Tensor, k: Tensor, v: Tensor, beta: Tensor, state: 
     mask = _active_mask(active, ("b",), dims, q.device)
     o = torch.empty_like(q)
     entry = "vsp_delta_step_f32" if dtype == torch.float32 else "vsp_delta_step_bf16"
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         _lib.call(entry, q.data_ptr(), k.data_ptr(), v.data_ptr(), beta.data_ptr(), state.data_ptr(),
                   out_state.data_ptr(), o.data_ptr(), _lib.ptr(mask), b, h, dk, _lib.stream_of(q.device))
     return o, out_state
@@ -380,7 +380,7 @@ def delta_scan_step_keys(q: Tensor, z: Tensor, v: Tensor, beta: Tensor, history:
             raise ContractError(f"{name} must be 16-byte aligned")
     mask = _active_mask(active, ("b",), dims, q.device)
     o = torch.empty_like(q)
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         _lib.call("vsp_delta_step_keys_bf16", q.data_ptr(), zc.data_ptr(), v.data_ptr(), beta.data_ptr(),
                   history.data_ptr() if width > 1 else None, tc.data_ptr(), width, state.data_ptr(),
                   out_state.data_ptr(), o.data_ptr(), _lib.ptr(mask), b, h, dk, _lib.stream_of(q.device))
@@ -421,7 +421,7 @@ class _WriteStrength(torch.autograd.Function):
         beta = torch.empty_like(lg)
         rows = lg.numel() // lg.shape[-1] if lg.dim() else 1
         entry = "vsp_write_strength_f32" if lg.dtype == torch.float32 else "vsp_write_strength_bf16"
-        with torch.cuda.device(lg.device):
+        with _lib.on_device(lg.device):
             _lib.call(entry, lg.data_ptr(), _lib.ptr(mm), float(alpha), beta.data_ptr(), rows, lg.shape[-1],
                       _lib.stream_of(lg.device))
         ctx.save_for_backward(beta, *(() if mm is None else (mm,)))
@@ -501,7 +501,7 @@ def delta_scan_fused_logits(q: Tensor, k: Tensor, v: Tensor, logits: Tensor, sta
     ws_bytes = int(lib.vsp_delta_scan_workspace_bytes(b, n, h, dk, int(fp32)))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     entry = "vsp_delta_scan_logits_f32" if fp32 else "vsp_delta_scan_logits_bf16"
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         _lib.call(entry, q.data_ptr(), k.data_ptr(), v.data_ptr(), logits.data_ptr(), _lib.ptr(mm), a,
                   state.data_ptr(), o.data_ptr(), s_out.data_ptr(), _lib.ptr(ws), ws_bytes, _lib.ptr(mask),
                   b, n, h, dk, _lib.stream_of(q.device))

@@ -70,7 +70,7 @@ def _check(z: Tensor, history: Tensor, taps: Tensor, heads: int) -> tuple[int, i
 class _FusedKeys(torch.autograd.Function):
     @staticmethod
     def forward(ctx: Any, z: Tensor, history: Tensor, taps: Tensor, heads: int) -> Tensor:  # noqa: D102
-        b, n, d, width = _check(z, history, taps, heads)
+        (b, n, d), width = z.shape, int(taps.shape[0])  # fused_keys has checked the contract
         zc = _aligned(z)
         hist = _aligned(history.detach().to(torch.float32))
         wide = _aligned(taps.detach().to(torch.float32))
@@ -111,7 +111,7 @@ class _FusedKeys(torch.autograd.Function):
 
 def _key_step(z: Tensor, history: Tensor, taps: Tensor, heads: int, active: Tensor | None,
               carried_z: Tensor | None, want_history: bool, in_place: bool = False) -> tuple[Tensor, Tensor | None]:
-    b, n, d, width = _check(z, history, taps, heads)
+    (b, n, d), width = z.shape, int(taps.shape[0])  # the caller has checked the contract
     zc = _aligned(z)
     held = None if carried_z is None else _aligned(carried_z)
     flags = None if carried_z is None or active is None else active.contiguous().view(torch.uint8)
@@ -204,7 +204,7 @@ class _NormalizeKeys(torch.autograd.Function):
         x = _aligned(k.detach())
         y = torch.empty_like(x)
         width = x.shape[-1]
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             _lib.call(f"vsp_normalize_keys_{_SUFFIX[x.dtype]}", x.data_ptr(), y.data_ptr(), x.numel() // width,
                       width, _lib.stream_of(x.device))
         ctx.save_for_backward(x)
@@ -216,7 +216,7 @@ class _NormalizeKeys(torch.autograd.Function):
         g = _aligned(grad.to(x.dtype))
         gx = torch.empty_like(x)
         width = x.shape[-1]
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             _lib.call(f"vsp_normalize_keys_backward_{_SUFFIX[x.dtype]}", x.data_ptr(), g.data_ptr(), gx.data_ptr(),
                       x.numel() // width, width, _lib.stream_of(x.device))
         return gx

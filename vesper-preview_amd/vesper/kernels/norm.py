@@ -52,7 +52,7 @@ def rms_norm_bf16(x: Tensor, gain: Tensor | None = None, *, residual: Tensor | N
     if residual is None:
         if sum_out is not None:
             raise ContractError("sum_out needs a residual")
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             _lib.call("vsp_rms_norm_bf16", xc.data_ptr(), _lib.ptr(g), out.data_ptr(), rows, d,
                       _lib.stream_of(x.device))
         return out
@@ -68,7 +68,7 @@ def rms_norm_bf16(x: Tensor, gain: Tensor | None = None, *, residual: Tensor | N
             raise ContractError(f"sum_out: contiguous, aligned float32 {tuple(x.shape)} on {x.device}")
         if sum_out.data_ptr() == xc.data_ptr():
             raise ContractError("sum_out must not be x")
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         _lib.call("vsp_add_rms_norm_bf16", xc.data_ptr(), rc.data_ptr(), _lib.ptr(sum_out), _lib.ptr(g),
                   out.data_ptr(), rows, d, _lib.stream_of(x.device))
     return out
@@ -153,7 +153,7 @@ def decode_projection(x: Tensor, weights_t: Tensor, used: tuple[int, ...], *, re
     outs = [torch.empty(m, u, dtype=torch.bfloat16, device=x.device) for u in used]
     ptrs = [o.data_ptr() for o in outs] + [0] * (4 - p)
     widths = list(used) + [1] * (4 - p)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         _lib.call("vsp_decode_proj_bf16", xc.data_ptr(), _lib.ptr(rc), _lib.ptr(sum_out), _lib.ptr(gc), wc.data_ptr(),
                   p, cols, d, m, *widths, *ptrs, -1 if sigmoid_block is None else sigmoid_block,
                   _lib.ptr(rot_pos), _lib.ptr(rot_freq), rot_mask, rot_dk, _lib.stream_of(x.device))
@@ -203,7 +203,7 @@ def projection(z: Tensor, weights_t: Tensor, used: tuple[int, ...], *,
     outs = [torch.empty(m, u, dtype=torch.bfloat16, device=z.device) for u in used]
     ptrs = [o.data_ptr() for o in outs] + [0] * (4 - p)
     widths = list(used) + [1] * (4 - p)
-    with torch.cuda.device(z.device):
+    with _lib.on_device(z.device):
         _lib.call("vsp_project_bf16", zc.data_ptr(), wc.data_ptr(), p, cols, d, m, *widths, *ptrs,
                   -1 if sigmoid_block is None else sigmoid_block, _lib.stream_of(z.device))
     return outs

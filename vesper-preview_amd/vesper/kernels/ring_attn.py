@@ -142,7 +142,7 @@ def ring_attention(q: Tensor, k: Tensor, v: Tensor, pos: Tensor, cache: RingKVCa
     entry = "vsp_ring_attn_bf16" if q.dtype == torch.bfloat16 else "vsp_ring_attn_f16"
     if ring_dtype == torch.float32:
         entry += "_ring_f32"
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         _lib.call(entry, q.data_ptr(), k.data_ptr(), v.data_ptr(), pos.data_ptr(), ring.k.data_ptr(),
                   ring.v.data_ptr(), ring.pos.data_ptr(), ring.valid.data_ptr(), o.data_ptr(), _lib.ptr(mask),
                   counters.data_ptr(), counters.numel() * 4, b, h, hkv, dk, cache.window, 1.0 / math.sqrt(dk), 1,

@@ -55,7 +55,7 @@ class _WindowAttention(torch.autograd.Function):
         qc, kc, vc = _aligned(q.detach()), _aligned(keys.detach()), _aligned(values.detach())
         o = torch.empty_like(qc)
         args = (b, n, m, h, hkv, dk, int(window), scale, _lib.stream_of(q.device))
-        with torch.cuda.device(q.device):
+        with _lib.on_device(q.device):
             if any(ctx.needs_input_grad[:3]):
                 lse = torch.empty(b, h, n, dtype=torch.float32, device=q.device)
                 _lib.call(f"vsp_window_attn_lse_{suffix}", qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), o.data_ptr(),
@@ -79,7 +79,7 @@ class _WindowAttention(torch.autograd.Function):
         dq, dk_, dv = torch.empty_like(qc), torch.empty_like(kc), torch.empty_like(vc)
         workspace = torch.empty(b * h * n, dtype=torch.float32, device=qc.device)
         suffix = "bf16" if qc.dtype == torch.bfloat16 else "f16"
-        with torch.cuda.device(qc.device):
+        with _lib.on_device(qc.device):
             _lib.call(f"vsp_window_attn_backward_{suffix}", qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), o.data_ptr(),
                       go.data_ptr(), lse.data_ptr(), workspace.data_ptr(), dq.data_ptr(), dk_.data_ptr(), dv.data_ptr(),
                       b, n, m, h, hkv, dk, int(window), scale, _lib.stream_of(qc.device))
@@ -95,7 +95,7 @@ def _carried_call(q: Tensor, keys: Tensor, values: Tensor, carried: tuple[Tensor
     kh, vh = _aligned(carried[0]), _aligned(carried[1])
     o = torch.empty_like(qc)
     suffix = "bf16" if q.dtype == torch.bfloat16 else "f16"
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         _lib.call(f"vsp_window_attn_carried_{suffix}", qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), kh.data_ptr(),
                   vh.data_ptr(), o.data_ptr(), mask.data_ptr(), b, n, s - n, h, hkv, dk, int(window), scale,
                   _lib.stream_of(q.device))
@@ -212,7 +212,7 @@ def window_attention_cached(q: Tensor, cache_keys: Tensor, cache_values: Tensor,
     qc, ck, cv, kc, vc = (_aligned(t) for t in tensors)
     o = torch.empty_like(qc)
     suffix = "bf16" if q.dtype == torch.bfloat16 else "f16"
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         _lib.call(f"vsp_window_attn_cached_{suffix}", qc.data_ptr(), ck.data_ptr(), cv.data_ptr(), kc.data_ptr(),
                   vc.data_ptr(), o.data_ptr(), None, b, n, m, h, hkv, dk, int(window), 1.0 / math.sqrt(dk),
                   _lib.stream_of(q.device))
