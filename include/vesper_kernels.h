@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define VSP_ABI_VERSION 20
+#define VSP_ABI_VERSION 21
 
 /* Status codes. */
 #define VSP_OK 0
@@ -259,6 +259,12 @@ int vsp_window_attn_backward_f16(const void* q, const void* keys, const void* va
 int vsp_kv_cache_push(const void* cache_k, const void* cache_v, const int64_t* cache_pos, const void* k,
                       const void* v, const int64_t* pos, void* out_k, void* out_v, int64_t* out_pos, int B, int M,
                       int N, int HKV, int D, int elem_bytes, int window, void* stream);
+
+/* The attention's precondition (vesper/attention.py:377-379): *broken (device or pinned host memory, zero
+ * before) becomes 1 if any row's M cache positions and N chunk positions (int64, [B, M] and [B, N]) do
+ * not go up by one throughout. */
+int vsp_positions_consecutive(const int64_t* cache_pos, const int64_t* pos, int* broken, int B, int M, int N,
+                              void* stream);
 
 /* Rotary position embedding (vesper/attention.py:178-217, `rotary`, as `WindowedAttention.project`
  * applies it to q and k, attention.py:292): q [B, N, H, D] and k [B, N, HKV, D] (HKV may be 0 and

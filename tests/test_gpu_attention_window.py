@@ -206,3 +206,27 @@ def test_attend_refuses_positions_that_are_not_consecutive():
     k = torch.zeros(1, 4, 2, 16, dtype=BF16, device=GPU)
     with pytest.raises(ContractError, match="consecutive"):
         attend(q, k, k, torch.tensor([[0, 1, 3, 4]], device=GPU), kv_cache_empty(1, 2, 16, 8, BF16, GPU))
+
+
+@pytest.mark.parametrize(("m", "n"), [(0, 2), (1, 1), (63, 1), (1, 300), (64, 1000)])
+@pytest.mark.parametrize("where", ["first", "join", "last", "none"])
+def test_a_break_anywhere_in_the_positions_is_refused_and_the_next_call_runs(m, n, where):
+    from vesper.attention import KVCache, attend
+    from vesper.contracts import ContractError
+
+    b, w = 3, 64
+    g = torch.Generator().manual_seed(m + n)
+    q = torch.randn(b, n, 2, 16, generator=g).to(GPU, torch.bfloat16)
+    k, ck = (torch.randn(b, r, 1, 16, generator=g).to(GPU, torch.bfloat16) for r in (n, m))
+    pos = (torch.arange(m + n) + 5).expand(b, m + n).clone()
+    want = attend(q, k, k, pos[:, m:].to(GPU), KVCache(ck, ck, pos[:, :m].to(GPU), w))
+    at = {"first": 1, "join": max(m, 1), "last": m + n - 1}.get(where)
+    if at is not None:
+        pos[b - 1, at:] += 1  # one gap, in the last row
+    cache = KVCache(ck, ck, pos[:, :m].to(GPU), w)
+    if at is not None:
+        with pytest.raises(ContractError, match="consecutive"):
+            attend(q, k, k, pos[:, m:].to(GPU), cache)
+        return
+    o, after = attend(q, k, k, pos[:, m:].to(GPU), cache)
+    assert torch.equal(o, want[0]) and torch.equal(after.pos, want[1].pos)

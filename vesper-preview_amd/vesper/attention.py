@@ -241,9 +241,44 @@ def attend(q: Tensor, k: Tensor, v: Tensor, pos: Tensor, cache: KVCache) -> tupl
         return q.new_zeros(q.shape), cache
     if q.is_cuda and q.dtype not in WINDOW_KERNEL_DTYPES:
         return _attend_blocked(q, k, v, pos, cache), kv_cache_push(cache, k, v, pos)
-    kpos = torch.cat([cache.pos, pos], dim=1)
-    if kpos.shape[1] > 1:
-        require((kpos[:, 1:] - kpos[:, :-1] == 1).all().reshape(1), "attend: cache and chunk positions must be consecutive")
+    message = "attend: cache and chunk positions must be consecutive"
+    if not q.is_cuda or q.device != pos.device or q.device != cache.pos.device or torch.cuda.is_current_stream_capturing():
+        kpos = torch.cat([cache.pos, pos], dim=1)
+        if kpos.shape[1] > 1:
+            require((kpos[:, 1:] - kpos[:, :-1] == 1).all().reshape(1), message)
+        return _attend_window(q, k, v, pos, cache)
+    check = _PositionsCheck(cache.pos, pos)
+    try:
+        return _attend_window(q, k, v, pos, cache)
+    finally:
+        if check.broken():
+            raise ContractError(message)
+
+
+class _PositionsCheck:
+    """The check of the positions, queued ahead of the attention and read back after the attention and
+    the push are queued too: the host waits for the check's kernel alone, with the others behind it."""
+
+    def __init__(self, cache_pos: Tensor, pos: Tensor) -> None:
+        b, n = pos.shape
+        self.inputs = cache_pos.contiguous(), pos.contiguous()
+        self.word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self.done = torch.cuda.Event()
+        stream = torch.cuda.current_stream(pos.device)
+        with _lib.on_device(pos.device):
+            status = _lib.library().vsp_positions_consecutive(
+                self.inputs[0].data_ptr(), self.inputs[1].data_ptr(), self.word.data_ptr(), b, cache_pos.shape[1], n,
+                stream.cuda_stream)
+            self.done.record(stream)
+        if status != 0:
+            _lib.refuse("vsp_positions_consecutive", status)
+
+    def broken(self) -> bool:
+        self.done.synchronize()
+        return bool(self.word.item())
+
+
+def _attend_window(q: Tensor, k: Tensor, v: Tensor, pos: Tensor, cache: KVCache) -> tuple[Tensor, KVCache]:
     # the cache's rows and the chunk's as two sources of one kernel call (no concatenated copy)
     o = window_attention_cached(q, cache.k.to(q.dtype), cache.v.to(q.dtype), k.to(q.dtype), v.to(q.dtype),
                                 cache.window)

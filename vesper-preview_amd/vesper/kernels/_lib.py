@@ -19,7 +19,7 @@ import torch
 HERE = Path(__file__).resolve().parent
 LIBRARY_PATH = HERE / "libvesper_kernels.so"
 HEADER_PATH = HERE.parents[2] / "include" / "vesper_kernels.h"
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 P = ctypes.c_void_p
 I = ctypes.c_int
@@ -77,6 +77,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "vsp_key_step_f32": (I, [P, P, P, P, P, P, P, I, I, I, I, I, P]),
     "vsp_copy_rows_where": (I, [I, P, P, P, P, I, P]),
     "vsp_kv_cache_push": (I, [P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P]),
+    "vsp_positions_consecutive": (I, [P, P, P, I, I, I, P]),
     "vsp_rotary_qk_bf16": (I, [P, P, P, P, P, P, I, I, I, I, I, P]),
     "vsp_rotary_qk_f16": (I, [P, P, P, P, P, P, I, I, I, I, I, P]),
     "vsp_rotary_qk_f32": (I, [P, P, P, P, P, P, I, I, I, I, I, P]),
@@ -209,5 +210,10 @@ def call(name: str, *args: object) -> None:
         check_faults()
     status = getattr(lib, name)(*args)
     if status != 0:
-        message = lib.vsp_last_error().decode("utf-8", "replace")
-        raise KernelLibraryError(f"{name} returned {status}: {message}")
+        refuse(name, status)
+
+
+def refuse(name: str, status: int) -> None:
+    """Raise ``KernelLibraryError`` for an entry point's nonzero status."""
+    message = library().vsp_last_error().decode("utf-8", "replace")
+    raise KernelLibraryError(f"{name} returned {status}: {message}")
