@@ -463,6 +463,16 @@ def test_bf16_gradients_over_several_chunks_with_an_active_mask(dk):
     _grad_check(delta_scan_fused, _bf16_inputs(2, 300, 3, dk, seed=dk), TOL, active=act)
 
 
+@pytest.mark.parametrize("dk", [32, 64])
+@pytest.mark.parametrize("n", [16, 63, 64, 65, 81, 128])
+def test_bf16_gradients_at_the_edges_of_a_chunk(dk, n):
+    # one row block of 16 alone, and a 64-token chunk one under, whole and one over
+    from vesper.kernels.delta_scan import delta_scan_fused
+
+    act = torch.rand(3, n, generator=torch.Generator().manual_seed(n)) < 0.8
+    _grad_check(delta_scan_fused, _bf16_inputs(3, n, 5, dk, seed=n + dk), TOL, active=act)
+
+
 def test_bf16_gradients_at_width_128_over_several_chunks_with_an_active_mask():
     # width 128: the chunk kernel reads the states' fragments from the chains' records (both
     # orientations) instead of LDS tiles

@@ -788,7 +788,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   }
 }
 
-// ---- the chunk kernel on bf16 LDS tiles (bf16 entry, head widths 32 and 64) ------------------
+// ---- the chunk kernels on bf16 LDS tiles (bf16 entry, head widths 32, 64 and 128) --------------
 // Operands live in LDS as bf16 row-major tiles and feed 16x16x32 MFMAs in one of two forms, with
 // the same k order (k0 + 8 g + e for lane group g, element e) so that any two combine:
 // - frow(X, ld, r0, k0): row r0 + lq of X, k along its columns (one 16-byte read);
@@ -931,9 +931,7 @@ struct AccRows16 {
 // every other column tile from ch = w / 4. Products run over their full k range, unrolled: the
 // triangular factors hold exact zeros where they vanish, and straight-line code lets the compiler
 // issue a stage's LDS reads ahead of its MFMAs.
-// Threads of the bf16 chunk kernel: eight waves (two a SIMD, two tiles of every [64 x 64] product
-// each). Sixteen at width 64 (four a SIMD, one tile each) measured slower: the 128-register bound
-// of four waves a SIMD spilled (chunk kernel 115 -> 139 us at B8 T4096 H8 d64).
+// Width 128: eight waves (two a SIMD), one workgroup a CU.
 template <int D> struct ChunkShape {
   static constexpr int NTH = 512;
   static constexpr int NW = NTH / 64;
@@ -941,28 +939,21 @@ template <int D> struct ChunkShape {
 };
 
 template <int D>
-__global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_bf16_kernel(
+__global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_wide_bf16_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ k, const __bf16* __restrict__ v,
     const __bf16* __restrict__ beta, const __bf16* __restrict__ d_o, const uint8_t* __restrict__ active,
-    const float* __restrict__ ws, const __bf16* __restrict__ hrec, __bf16* __restrict__ dq, __bf16* __restrict__ dk,
+    const float* __restrict__ ws, __bf16* __restrict__ dq, __bf16* __restrict__ dk,
     __bf16* __restrict__ dv, __bf16* __restrict__ dbeta, int N, int H, int NC, int total) {
   using T = __bf16;
   constexpr int NT = D / 16;  // column tiles of a [64 x D] result
   constexpr int NTH = ChunkShape<D>::NTH, NCH = ChunkShape<D>::NCH;
-  // pitches: [64][D] and [D][D], [64][64]; up to D 64 rows 40 banks apart (the row fragments'
-  // 16-byte reads then meet no bank twice: each two groups of eight lanes in one cycle cover the 64
-  // banks), at D 128 (LDS-bound) 68
-  constexpr int LD = D <= 64 ? D + 16 : D + 8, L6 = D <= 64 ? kC + 16 : kC + 8;
-  // Up to D 64 the states H and G are LDS tiles. At D 128 they would not fit: their fragments come
-  // from the chains' records in global memory (column order for H and G as B operands, the
-  // transposed records for H^T and G^T), whose k order within 32 is 4 g .. 4 g + 3 of each 16-row
-  // tile, so the A operands they meet are read in that order too (frow2); and -dR goes over R.
-  constexpr bool kHGinLDS = D <= 64;
+  constexpr int LD = D + 8, L6 = kC + 8;  // pitches of [64][D] and [64][64] tiles
+  // The states H and G would not fit LDS: their fragments come from the chains' records in global
+  // memory (column order for H and G as B operands, the transposed records for H^T and G^T), whose k
+  // order within 32 is 4 g .. 4 g + 3 of each 16-row tile, so the A operands they meet are read in
+  // that order too (frow2); and -dR goes over R. Column tiles are not unrolled, for the registers.
   __shared__ __align__(16) T sQ[kC * LD], sK[kC * LD], sO[kC * LD], sR[kC * LD], sD[kC * LD], sDD[kC * LD];
-  __shared__ __align__(16) T sDRx[kHGinLDS ? kC * LD : 1];
-  __shared__ __align__(16) T sH[kHGinLDS ? D * LD : 1], sG[kHGinLDS ? D * LD : 1];
-  T* sDR = kHGinLDS ? sDRx : sR;
-  constexpr int kU = kHGinLDS ? NT / NCH : 1;  // column tiles unrolled (D 128: one, for the registers)
+  T* sDR = sR;
   __shared__ __align__(16) T sT[kC * L6], sL[kC * L6], sP[kC * L6], sM[kC * L6];
   __shared__ float sB[kC], sPart[4 * kC], sRow[NCH * kC];
   T* sX1 = sT;   // X1 = L^T dL once T is done with
@@ -971,10 +962,8 @@ __global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_bf16_kernel
   // wave w: column group ch = w / 4 and row block rb; the waves of one SIMD (w, w + 4, ...) take
   // row blocks rb and 3 - rb in turn, which evens out the triangular products' work
   const int w = threadIdx.x >> 6, ch = w >> 2, rb = (ch & 1) == 0 ? (w & 3) : 3 - (w & 3), r0 = 16 * rb;
-  // A workgroup walks chunks blockIdx.x, + gridDim.x, ...: the next chunk's operands are loaded
-  // into registers while the current one is computed.
+  // A workgroup walks chunks blockIdx.x, + gridDim.x, ...
   ChunkRows16<D, NTH> rq, rk, ro, rv;
-  AccRows16<kHGinLDS ? D : 16, NTH> mh, mg;
   ChunkBeta<T> rbeta;
   bf16x8 lraw;
   auto fetch = [&](int cid) {
@@ -987,18 +976,10 @@ __global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_bf16_kernel
     rk.fetch(k, b, h, t0, N, H);
     ro.fetch(d_o, b, h, t0, N, H, active);
     rv.fetch(v, b, h, t0, N, H);
-    if constexpr (kHGinLDS) {
-      // the chunk's starting state: the forward's record when it kept one, else the chain's
-      mh.fetch(hrec != nullptr ? hrec + (size_t)cid * (D * D)
-                               : reinterpret_cast<const T*>(Ws<D>::Hs(const_cast<float*>(ws), cid)));
-      mg.fetch(reinterpret_cast<const T*>(Ws<D>::dHs(const_cast<float*>(ws), cid)));
-    }
     rbeta.fetch(beta, b, h, t0, N, H);
   };
-  // (at D 128 the registers go to the states' fragments: each chunk loads its own operands)
-  if constexpr (kHGinLDS) fetch(blockIdx.x);
   for (int cid = blockIdx.x; cid < total; cid += gridDim.x) {
-  if constexpr (!kHGinLDS) fetch(cid);
+  fetch(cid);
   const int c = cid % NC, bh = cid / NC;
   const int b = bh / H, h = bh - b * H;
   const int t0 = c * kC;
@@ -1006,39 +987,26 @@ __global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_bf16_kernel
   const T* gH = reinterpret_cast<const T*>(Ws<D>::Hs(const_cast<float*>(ws), cid));
   const T* gG = reinterpret_cast<const T*>(Ws<D>::dHs(const_cast<float*>(ws), cid));
   const int lane = threadIdx.x & 63;
-  auto bcol = [&](const T* rec, const T* tile, int ct, int kk) -> bf16x8 {
-    if constexpr (kHGinLDS) {
-      return fcol(tile, LD, 16 * ct, kk);
-    } else {
-      return *reinterpret_cast<const bf16x8*>(rec + accfrag2<NT>(ct, kk / 16, lane));  // tiles kk/16, +1
-    }
+  auto bcol = [&](const T* rec, int ct, int kk) -> bf16x8 {
+    return *reinterpret_cast<const bf16x8*>(rec + accfrag2<NT>(ct, kk / 16, lane));  // tiles kk/16, +1
   };
-  auto brow = [&](const T* rec, const T* tile, int ct, int kk) -> bf16x8 {
-    if constexpr (kHGinLDS) {
-      return frow(tile, LD, 16 * ct, kk);
-    } else {
-      const T* rr = rec + Ws<D>::kS;  // the transposed record
-      const bf16x4 lo = *reinterpret_cast<const bf16x4*>(rr + accfrag<NT>(kk / 16, ct, lane));
-      const bf16x4 hi = *reinterpret_cast<const bf16x4*>(rr + accfrag<NT>(kk / 16 + 1, ct, lane));
-      return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-    }
+  auto brow = [&](const T* rec, int ct, int kk) -> bf16x8 {
+    const T* rr = rec + Ws<D>::kS;  // the transposed record
+    const bf16x4 lo = *reinterpret_cast<const bf16x4*>(rr + accfrag<NT>(kk / 16, ct, lane));
+    const bf16x4 hi = *reinterpret_cast<const bf16x4*>(rr + accfrag<NT>(kk / 16 + 1, ct, lane));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
-  auto arow = [&](const T* X, int kk) -> bf16x8 { return kHGinLDS ? frow(X, LD, r0, kk) : frow2(X, LD, r0, kk); };
+  auto arow = [&](const T* X, int kk) -> bf16x8 { return frow2(X, LD, r0, kk); };
   {
     rq.put(sQ, LD);
     rk.put(sK, LD);
     ro.put(sO, LD);
     rv.put(sR, LD);
-    if constexpr (kHGinLDS) {
-      mh.put(sH, LD);
-      mg.put(sG, LD);
-    }
     if (threadIdx.x < kC * kC / 8) *reinterpret_cast<bf16x8*>(sL + (threadIdx.x >> 3) * L6 + 8 * (threadIdx.x & 7)) = lraw;
     rbeta.put(sB, t0, N);
   }
   static_assert(NTH * 8 >= kC * kC, "one 16-byte piece of L a thread at most");
   __syncthreads();
-  if constexpr (kHGinLDS) fetch(min(cid + (int)gridDim.x, total - 1));  // (the last chunk again past the end)
   // T = L diag(beta)
   for (int e = threadIdx.x; e < kC * kC / 8; e += NTH) {
     const int i = e / (kC / 8), j = 8 * (e % (kC / 8));
@@ -1048,12 +1016,12 @@ __global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_bf16_kernel
     *reinterpret_cast<bf16x8*>(sT + i * L6 + j) = x;
   }
   // R = V - K H in place (each lane reads only its own V entries)
-#pragma unroll kU
+#pragma unroll 1
   for (int u_ = 0; u_ < NT / NCH; ++u_) {
     const int ct = ch + NCH * u_;
     f32x4 acc = zero4();
     #pragma unroll
-    for (int kk = 0; kk < D; kk += 32) acc = mma32(arow(sK, kk), bcol(gH, sH, ct, kk), acc);
+    for (int kk = 0; kk < D; kk += 32) acc = mma32(arow(sK, kk), bcol(gH, ct, kk), acc);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       T& x = sR[(r0 + tile_row(r)) * LD + 16 * ct + tile_col()];
@@ -1074,14 +1042,14 @@ __global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_bf16_kernel
   }
   __syncthreads();
   // Delta = T R; dDelta = K G + P^T dO
-#pragma unroll kU
+#pragma unroll 1
   for (int u_ = 0; u_ < NT / NCH; ++u_) {
     const int ct = ch + NCH * u_;
     f32x4 d = zero4(), dd = zero4();
     #pragma unroll
     for (int kk = 0; kk < kC; kk += 32) d = mma32(frow(sT, L6, r0, kk), fcol(sR, LD, 16 * ct, kk), d);
     #pragma unroll
-    for (int kk = 0; kk < D; kk += 32) dd = mma32(arow(sK, kk), bcol(gG, sG, ct, kk), dd);
+    for (int kk = 0; kk < D; kk += 32) dd = mma32(arow(sK, kk), bcol(gG, ct, kk), dd);
     #pragma unroll
     for (int kk = 0; kk < kC; kk += 32) dd = mma32(fcol(sP, L6, r0, kk), fcol(sO, LD, 16 * ct, kk), dd);
     put_tile(sD, LD, r0, 16 * ct, d);
@@ -1116,8 +1084,8 @@ __global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_bf16_kernel
     put_tile(sS2, L6, r0, 16 * ct, s2);
     put_tile(sDL, L6, r0, 16 * ct, dt);
   }
-  if constexpr (!kHGinLDS) __syncthreads();
-#pragma unroll kU
+  __syncthreads();
+#pragma unroll 1
   for (int u_ = 0; u_ < NT / NCH; ++u_) {
     const int ct = ch + NCH * u_;
     f32x4 acc = zero4();
@@ -1128,12 +1096,12 @@ __global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_bf16_kernel
   }
   __syncthreads();
   // dQ = dO H^T + S2 K; X1 = L^T dL over T (L^T upper, dL lower: k from max(rb, ct))
-#pragma unroll kU
+#pragma unroll 1
   for (int u_ = 0; u_ < NT / NCH; ++u_) {
     const int ct = ch + NCH * u_;
     f32x4 acc = zero4();
     #pragma unroll
-    for (int kk = 0; kk < D; kk += 32) acc = mma32(arow(sO, kk), brow(gH, sH, ct, kk), acc);
+    for (int kk = 0; kk < D; kk += 32) acc = mma32(arow(sO, kk), brow(gH, ct, kk), acc);
     #pragma unroll
     for (int kk = 0; kk < kC; kk += 32) acc = mma32(frow(sS2, L6, r0, kk), fcol(sK, LD, 16 * ct, kk), acc);
     store_rows<T, D>(dq, b, h, t0, N, H, r0, 16 * ct, acc);
@@ -1177,14 +1145,14 @@ __global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_bf16_kernel
   }
   __syncthreads();
   // dK = Delta G^T + S2^T Q - dR H^T + M K + M^T K
-#pragma unroll kU
+#pragma unroll 1
   for (int u_ = 0; u_ < NT / NCH; ++u_) {
     const int ct = ch + NCH * u_;
     f32x4 acc = zero4();
     #pragma unroll
     for (int kk = 0; kk < D; kk += 32) {
-      acc = mma32(arow(sD, kk), brow(gG, sG, ct, kk), acc);
-      acc = mma32(arow(sDR, kk), brow(gH, sH, ct, kk), acc);
+      acc = mma32(arow(sD, kk), brow(gG, ct, kk), acc);
+      acc = mma32(arow(sDR, kk), brow(gH, ct, kk), acc);
     }
     #pragma unroll
     for (int kk = 0; kk < kC; kk += 32) {
@@ -1204,6 +1172,258 @@ __global__ __launch_bounds__(ChunkShape<D>::NTH) void scan_bwd_chunk_bf16_kernel
     dbeta[((size_t)b * N + t0 + i) * H + h] = (T)x;
   }
   __syncthreads();  // every read of this chunk's LDS is done before the next one is put
+  }
+}
+
+// Widths 32 and 64. Two workgroups of eight waves a CU: eight [64][72] tiles (74 KB), each reused as its
+// contents go dead, so one workgroup's barriers and LDS latency pass under the other's work. The kernel
+// is bound by that latency (thirteen chained products of 64^3 on a chunk, each a few MFMAs a wave): one
+// workgroup a CU with every operand in a tile of its own (133 KB, six barriers a chunk against ten)
+// and the next chunk's loads in registers took 93.4 us at B16 T1024 H12
+// d64 and this takes 77.5 (47 for its 250 MB at a large copy's rate).
+//   tile   holds in turn
+//   sQ     Q
+//   sK     K
+//   sO     dO, then X1 = L^T dL
+//   sR     V, R = V - K H, then dL = tril(dDelta R^T) diag(beta), then M = diag(beta) dA
+//   sH     H
+//   sG     G, then dDelta, then -dR
+//   sL     L
+//   sX     P = tril(Q K^T), then Delta, then S2 = tril(dO Delta^T)
+// dQ and dK accumulate in registers from the stage whose operands are there to the one that ends them.
+// T = L diag(beta) is formed in the fragments (rounded to bf16, as a tile of it would be).
+template <int D>
+__global__ __launch_bounds__(512, 4) void scan_bwd_chunk_bf16_kernel(
+    const __bf16* __restrict__ q, const __bf16* __restrict__ k, const __bf16* __restrict__ v,
+    const __bf16* __restrict__ beta, const __bf16* __restrict__ d_o, const uint8_t* __restrict__ active,
+    const float* __restrict__ ws, const __bf16* __restrict__ hrec, __bf16* __restrict__ dq, __bf16* __restrict__ dk,
+    __bf16* __restrict__ dv, __bf16* __restrict__ dbeta, int N, int H, int NC) {
+  using T = __bf16;
+  constexpr int NT = D / 16, NTH = 512, NCH = 2, U = NT / NCH;  // column tiles; a wave's share of a [64 x D] result
+  constexpr int LD = D + 8, L6 = kC + 8;                        // pitches of [.][D] and [64][64] tiles
+  static_assert(U >= 1 && LD <= L6, "widths 32 and 64");
+  __shared__ __align__(16) T sQ[kC * LD], sK[kC * LD], sH[D * LD], sG[kC * LD];
+  __shared__ __align__(16) T sO[kC * L6], sR[kC * L6], sL[kC * L6], sX[kC * L6];
+  __shared__ float sB[kC], sPart[4 * kC], sRow[NCH * kC];
+  const int w = threadIdx.x >> 6, ch = w >> 2, rb = ch == 0 ? w : 7 - w, r0 = 16 * rb;
+  const int c = blockIdx.x % NC, bh = blockIdx.x / NC;
+  const int b = bh / H, h = bh - b * H;
+  const int t0 = c * kC;
+  const size_t chunk = blockIdx.x;
+  {
+    ChunkRows16<D, NTH> rq, rk, ro, rv;
+    AccRows16<D, NTH> mh, mg;
+    ChunkBeta<T> rbeta;
+    rk.fetch(k, b, h, t0, N, H);
+    rv.fetch(v, b, h, t0, N, H);
+    rq.fetch(q, b, h, t0, N, H);
+    ro.fetch(d_o, b, h, t0, N, H, active);
+    // the chunk's starting state: the forward's record when it kept one, else the chain's
+    mh.fetch(hrec != nullptr ? hrec + chunk * (D * D) : reinterpret_cast<const T*>(Ws<D>::Hs(const_cast<float*>(ws), chunk)));
+    mg.fetch(reinterpret_cast<const T*>(Ws<D>::dHs(const_cast<float*>(ws), chunk)));
+    const T* gL = reinterpret_cast<const T*>(Ws<D>::L(const_cast<float*>(ws), chunk));
+    const bf16x8 lraw = *reinterpret_cast<const bf16x8*>(gL + 8 * threadIdx.x);  // [64][64]: eight elements a thread
+    rbeta.fetch(beta, b, h, t0, N, H);
+    rk.put(sK, LD);
+    rv.put(sR, LD);
+    rq.put(sQ, LD);
+    ro.put(sO, LD);
+    mh.put(sH, LD);
+    mg.put(sG, LD);
+    *reinterpret_cast<bf16x8*>(sL + (threadIdx.x >> 3) * L6 + 8 * (threadIdx.x & 7)) = lraw;
+    rbeta.put(sB, t0, N);
+  }
+  static_assert(NTH * 8 == kC * kC, "one 16-byte piece of L a thread");
+  __syncthreads();
+  // R = V - K H in place (each lane reads only its own V entries); P = tril(Q K^T), diagonal included
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int ct = ch + NCH * u;
+    f32x4 acc = zero4();
+#pragma unroll
+    for (int kk = 0; kk < D; kk += 32) acc = mma32(frow(sK, LD, r0, kk), fcol(sH, LD, 16 * ct, kk), acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      T& x = sR[(r0 + tile_row(r)) * LD + 16 * ct + tile_col()];
+      x = (T)((float)x - acc[r]);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int ct = ch + NCH * u;
+    f32x4 acc = zero4();
+    if (ct <= rb)
+#pragma unroll
+      for (int kk = 0; kk < D; kk += 32) acc = mma32(frow(sQ, LD, r0, kk), frow(sK, LD, 16 * ct, kk), acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = 16 * ct + tile_col() <= r0 + tile_row(r) ? acc[r] : 0.f;
+    put_tile(sX, L6, r0, 16 * ct, acc);
+  }
+  __syncthreads();
+  // Delta = T R over P; dDelta = K G + P^T dO, kept until G has been read
+  f32x4 dd[U], dka[U], dqa[U];
+  {
+    bf16x8 tf[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      tf[kk] = frow(sL, L6, r0, 32 * kk);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) tf[kk][e] = (T)((float)tf[kk][e] * sB[32 * kk + 8 * ((threadIdx.x & 63) >> 4) + e]);
+    }
+    f32x4 d[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int ct = ch + NCH * u;
+      d[u] = dd[u] = zero4();
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) d[u] = mma32(tf[kk], fcol(sR, LD, 16 * ct, 32 * kk), d[u]);
+#pragma unroll
+      for (int kk = 0; kk < D; kk += 32) dd[u] = mma32(frow(sK, LD, r0, kk), fcol(sG, LD, 16 * ct, kk), dd[u]);
+#pragma unroll
+      for (int kk = 0; kk < kC; kk += 32) dd[u] = mma32(fcol(sX, L6, r0, kk), fcol(sO, LD, 16 * ct, kk), dd[u]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) put_tile(sX, LD, r0, 16 * (ch + NCH * u), d[u]);
+  }
+  __syncthreads();
+  // dK = Delta G^T; then dDelta over G; meanwhile S2 = tril(dO Delta^T) and dQ = dO H^T, kept
+  f32x4 s2[2];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int ct = ch + NCH * u;
+    dka[u] = dqa[u] = zero4();
+#pragma unroll
+    for (int kk = 0; kk < D; kk += 32) dka[u] = mma32(frow(sX, LD, r0, kk), frow(sG, LD, 16 * ct, kk), dka[u]);
+#pragma unroll
+    for (int kk = 0; kk < D; kk += 32) dqa[u] = mma32(frow(sO, LD, r0, kk), frow(sH, LD, 16 * ct, kk), dqa[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int ct = ch + NCH * u;
+    s2[u] = zero4();
+    if (ct <= rb)
+#pragma unroll
+      for (int kk = 0; kk < D; kk += 32) s2[u] = mma32(frow(sO, LD, r0, kk), frow(sX, LD, 16 * ct, kk), s2[u]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s2[u][r] = 16 * ct + tile_col() <= r0 + tile_row(r) ? s2[u][r] : 0.f;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; ++u) put_tile(sG, LD, r0, 16 * (ch + NCH * u), dd[u]);
+#pragma unroll
+  for (int u = 0; u < 2; ++u) put_tile(sX, L6, r0, 16 * (ch + NCH * u), s2[u]);
+  __syncthreads();
+  // dT = dDelta R^T: dbeta_j gets sum_i dT_ij L_ij (column sums per row block into sPart), dL =
+  // tril(dT) diag(beta); dR = T^T dDelta (= dV), kept negated for dK
+  {
+    f32x4 dl[2], dr[U];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int ct = ch + NCH * u;
+      f32x4 dt = zero4();
+      if (ct <= rb)
+#pragma unroll
+        for (int kk = 0; kk < D; kk += 32) dt = mma32(frow(sG, LD, r0, kk), frow(sR, LD, 16 * ct, kk), dt);
+      const int j = 16 * ct + tile_col();
+      float part = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = r0 + tile_row(r);
+        part += dt[r] * (float)sL[i * L6 + j];
+        dl[u][r] = j <= i ? dt[r] * sB[j] : 0.f;
+      }
+      part = sum_over_rows(part);
+      if ((threadIdx.x & 63) < 16) sPart[rb * kC + j] = part;
+    }
+    bf16x8 tf[2];  // columns r0 + lq of T
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      tf[kk] = fcol(sL, L6, r0, 32 * kk);
+      const float bs = sB[r0 + (threadIdx.x & 15)];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) tf[kk][e] = (T)((float)tf[kk][e] * bs);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int ct = ch + NCH * u;
+      dr[u] = zero4();
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) dr[u] = mma32(tf[kk], fcol(sG, LD, 16 * ct, 32 * kk), dr[u]);
+      store_rows<T, D>(dv, b, h, t0, N, H, r0, 16 * ct, dr[u]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) put_tile(sG, LD, r0, 16 * (ch + NCH * u), -dr[u]);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) put_tile(sR, L6, r0, 16 * (ch + NCH * u), dl[u]);
+  }
+  __syncthreads();
+  // dQ += S2 K, dK += S2^T Q - dR H^T; X1 = L^T dL over dO
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int ct = ch + NCH * u;
+#pragma unroll
+    for (int kk = 0; kk < kC; kk += 32) dqa[u] = mma32(frow(sX, L6, r0, kk), fcol(sK, LD, 16 * ct, kk), dqa[u]);
+    store_rows<T, D>(dq, b, h, t0, N, H, r0, 16 * ct, dqa[u]);
+#pragma unroll
+    for (int kk = 0; kk < D; kk += 32) dka[u] = mma32(frow(sG, LD, r0, kk), frow(sH, LD, 16 * ct, kk), dka[u]);
+#pragma unroll
+    for (int kk = 0; kk < kC; kk += 32) dka[u] = mma32(fcol(sX, L6, r0, kk), fcol(sQ, LD, 16 * ct, kk), dka[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int ct = ch + NCH * u;
+    f32x4 x1 = zero4();
+#pragma unroll
+    for (int kk = 0; kk < kC; kk += 32) x1 = mma32(fcol(sL, L6, r0, kk), fcol(sR, L6, 16 * ct, kk), x1);
+    put_tile(sO, L6, r0, 16 * ct, x1);
+  }
+  __syncthreads();
+  // dA = -tril(X1 L^T, -1) (L^T[k][j] nonzero for k <= j); dbeta_i gets sum_m dA_im (k_i . k_m)
+  // (row sums per column half into sRow); M = diag(beta) dA over dL
+  float rows[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int ct = ch + NCH * u;
+    f32x4 da = zero4(), gk = zero4();
+    if (ct <= rb) {
+#pragma unroll
+      for (int kk = 0; kk < kC; kk += 32) da = mma32(frow(sO, L6, r0, kk), frow(sL, L6, 16 * ct, kk), da);
+#pragma unroll
+      for (int kk = 0; kk < D; kk += 32) gk = mma32(frow(sK, LD, r0, kk), frow(sK, LD, 16 * ct, kk), gk);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = r0 + tile_row(r), j = 16 * ct + tile_col();
+      da[r] = j < i ? -da[r] : 0.f;
+      rows[r] += da[r] * gk[r];
+      da[r] *= sB[i];
+    }
+    put_tile(sR, L6, r0, 16 * ct, da);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float x = group_sum<16>(rows[r]);
+    if (tile_col() == 0) sRow[ch * kC + r0 + tile_row(r)] = x;
+  }
+  __syncthreads();
+  // dK += M K + M^T K
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int ct = ch + NCH * u;
+#pragma unroll
+    for (int kk = 0; kk < kC; kk += 32) {
+      const bf16x8 kc = fcol(sK, LD, 16 * ct, kk);
+      dka[u] = mma32(fcol(sR, L6, r0, kk), kc, dka[u]);
+      dka[u] = mma32(frow(sR, L6, r0, kk), kc, dka[u]);
+    }
+    store_rows<T, D>(dk, b, h, t0, N, H, r0, 16 * ct, dka[u]);
+  }
+  const int i = threadIdx.x;
+  if (i < kC && t0 + i < N) {
+    const float x = ((sPart[i] + sPart[kC + i]) + (sPart[2 * kC + i] + sPart[3 * kC + i])) + (sRow[i] + sRow[kC + i]);
+    dbeta[((size_t)b * N + t0 + i) * H + h] = (T)x;
   }
 }
 
@@ -1453,10 +1673,13 @@ void launch(const TIn* q, const TIn* k, const TIn* v, const TIn* beta, const flo
   }
   hipLaunchKernelGGL((scan_bwd_chains_kernel<TIn, D>), dim3(hrec != nullptr ? slices : 2 * slices), dim3(64), 0, stream,
                      state_in, d_state, d_state_in, ws, NC, (int)slices, hrec != nullptr ? (int)slices : 0);
-  if constexpr (sizeof(TIn) == 2 && D >= 32)
-    hipLaunchKernelGGL((scan_bwd_chunk_bf16_kernel<D>), dim3(min(chunks, persistent_blocks(1))),
-                       dim3(ChunkShape<D>::NTH), 0, stream, q, k, v, beta, d_o, active, ws, hrec, dq, dk, dv, dbeta, N, H,
-                       NC, (int)chunks);
+  if constexpr (sizeof(TIn) == 2 && D >= 128)
+    hipLaunchKernelGGL((scan_bwd_chunk_wide_bf16_kernel<D>), dim3(min(chunks, persistent_blocks(1))),
+                       dim3(ChunkShape<D>::NTH), 0, stream, q, k, v, beta, d_o, active, ws, dq, dk, dv, dbeta, N, H, NC,
+                       (int)chunks);
+  else if constexpr (sizeof(TIn) == 2 && D >= 32)
+    hipLaunchKernelGGL((scan_bwd_chunk_bf16_kernel<D>), dim3(chunks), dim3(512), 0, stream, q, k, v, beta, d_o, active,
+                       ws, hrec, dq, dk, dv, dbeta, N, H, NC);
   else
     hipLaunchKernelGGL((scan_bwd_chunk_kernel<TIn, D>), dim3(chunks), dim3(kChunkThreads), 0, stream, q, k, v, beta, d_o,
                        active, ws, dq, dk, dv, dbeta, N, H, NC);
