@@ -208,12 +208,17 @@ __device__ __forceinline__ size_t accfrag2(int s, int rt, int l) {
   else return ((size_t)(s * (NT / 2) + rt / 2) * 64 + l) * 8 + (rt & 1) * 4;
 }
 
-// Eight waves in the chunk kernel's arrangement: wave w owns row block rb (rb and 3 - rb on one
-// SIMD) and every other column tile from ch = w / 4; triangular zeros are skipped.
-constexpr int kPrepThreads = 512;
+// Waves in the chunk kernel's arrangement: wave w owns row block rb (the waves of one SIMD take rb and
+// 3 - rb in turn) and every NCH-th column tile from ch = w / 4; triangular zeros are skipped. One
+// workgroup's LDS fills a CU, so its waves alone hide LDS and MFMA latency: sixteen from width 32 up
+// (at 16 there is one column tile to share). With the chunk kernel's sixteen: float32 backward at B8 T1000
+// H8 d64 209 -> 189 us, B16 T1024 H8 d32 200 -> 187 (the chunk kernel's alone 197 and 190).
+constexpr int kPrepThreads = 512;  // the bf16 prep kernel's
+
+template <int D> constexpr int kPrepThreadsF = D >= 32 ? 1024 : 512;
 
 template <typename TIn, int D>
-__global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_kernel(const TIn* __restrict__ q, const TIn* __restrict__ k,
+__global__ __launch_bounds__(kPrepThreadsF<D>) void scan_bwd_prep_kernel(const TIn* __restrict__ q, const TIn* __restrict__ k,
                                                             const TIn* __restrict__ v, const TIn* __restrict__ beta,
                                                             const TIn* __restrict__ d_o,
                                                             const uint8_t* __restrict__ active,
@@ -226,9 +231,9 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_kernel(const TIn* 
   const int b = bh / H, h = bh - b * H;
   const int t0 = c * kC;
   const size_t chunk = blockIdx.x;
-  constexpr int NTH = kPrepThreads, NT = D / 16;
+  constexpr int NTH = kPrepThreadsF<D>, NT = D / 16, NCH = NTH / 256;
   constexpr bool BF = sizeof(TIn) == 2;  // bf16 inputs: the products on bf16 MFMA (fp32 accumulation)
-  const int w = threadIdx.x >> 6, ch = w >> 2, rb = ch == 0 ? w : 7 - w, r0 = 16 * rb;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ch = w >> 2, rb = (ch & 1) == 0 ? (w & 3) : 3 - (w & 3), r0 = 16 * rb;
   {
     ChunkRows<TIn, D, NTH> rk, rq, ro, rv;
     ChunkBeta<TIn> rbeta;
@@ -245,7 +250,7 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_kernel(const TIn* 
   }
   __syncthreads();
   // A = tril(diag(beta) K K^T, -1) (tiles above the diagonal: zeros)
-  for (int ct = ch; ct < 4; ct += 2) {
+  for (int ct = ch; ct < 4; ct += NCH) {
     const f32x4 acc = ct <= rb ? mm16<false, true, BF>(sK + r0 * PD, PD, sK + 16 * ct * PD, PD, D, zero4()) : zero4();
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -301,7 +306,7 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_kernel(const TIn* 
   for (int e = threadIdx.x; e < kC * kC / 4; e += NTH)
     *reinterpret_cast<f32x4*>(gL + 4 * e) = *reinterpret_cast<const f32x4*>(sL + (e / (kC / 4)) * kPC + 4 * (e % (kC / 4)));
   // W = L diag(beta) K and U = L diag(beta) V (L lower triangular: k blocks 0 .. rb)
-  for (int ct = ch; ct < NT; ct += 2) {
+  for (int ct = ch; ct < NT; ct += NCH) {
     const f32x4 aw = mm16k<false, false, BF>(sL + r0 * kPC, kPC, sK + 16 * ct, PD, 0, rb + 1, zero4(), sB);
     const f32x4 au = mm16k<false, false, BF>(sL + r0 * kPC, kPC, sV + 16 * ct, PD, 0, rb + 1, zero4(), sB);
 #pragma unroll
@@ -312,7 +317,7 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_kernel(const TIn* 
     }
   }
   // P = tril(Q K^T), diagonal included, into sA (tiles above the diagonal: zeros)
-  for (int ct = ch; ct < 4; ct += 2) {
+  for (int ct = ch; ct < 4; ct += NCH) {
     const f32x4 acc = ct <= rb ? mm16<false, true, BF>(sQ + r0 * PD, PD, sK + 16 * ct * PD, PD, D, zero4()) : zero4();
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -322,7 +327,7 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_kernel(const TIn* 
   }
   __syncthreads();  // sW, sA complete; sV's reads are done
   // Z = P^T dO into sV (P^T upper triangular: k blocks rb .. 3)
-  for (int ct = ch; ct < NT; ct += 2) {
+  for (int ct = ch; ct < NT; ct += NCH) {
     const f32x4 acc = mm16k<true, false, BF>(sA + r0, kPC, sO + 16 * ct, PD, rb, 4, zero4());
 #pragma unroll
     for (int r = 0; r < 4; ++r) sV[(r0 + tile_row(r)) * PD + 16 * ct + tile_col()] = acc[r];
@@ -569,29 +574,30 @@ __global__ __launch_bounds__(64) void scan_bwd_chains_kernel(const float* __rest
   }
 }
 
-// Eight waves, two per SIMD, hiding each other's LDS and MFMA latency: wave w owns row block rb
-// of every [64 x .] result and every other column tile from ch = w / 4. Waves w and w + 4 (one
-// SIMD) own row blocks rb and 3 - rb: the triangular products (whose tiles and k ranges grow with
-// the row block) then load every SIMD about evenly. Tiles that a triangular factor makes zero are
-// not computed, and each product runs over the k blocks its triangular operand leaves nonzero.
-constexpr int kChunkThreads = 512;
+// Sixteen waves, four per SIMD, hiding each other's LDS and MFMA latency (eight at width 16): wave w
+// owns row block rb of every [64 x .] result and every NCH-th column tile from ch = w / 4. The waves of
+// one SIMD (w, w + 4, ...) own row blocks rb and 3 - rb in turn: the triangular products (whose tiles
+// and k ranges grow with the row block) then load every SIMD about evenly. Tiles that a triangular
+// factor makes zero are not computed, and each product runs over the k blocks its triangular operand
+// leaves nonzero.
+template <int D> constexpr int kChunkThreads = D >= 32 ? 1024 : 512;
 
 template <typename TIn, int D>
-__global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
+__global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
     const TIn* __restrict__ q, const TIn* __restrict__ k, const TIn* __restrict__ v, const TIn* __restrict__ beta,
     const TIn* __restrict__ d_o, const uint8_t* __restrict__ active, const float* __restrict__ ws,
     TIn* __restrict__ dq, TIn* __restrict__ dk, TIn* __restrict__ dv, TIn* __restrict__ dbeta, int N, int H, int NC) {
   constexpr int P = kPC;  // every buffer is [64][68]
-  constexpr int NT = D / 16, NTW = (NT + 1) / 2;  // column tiles of a [64 x D] result; a wave's share
-  constexpr int NTH = kChunkThreads;
+  constexpr int NTH = kChunkThreads<D>, NCH = NTH / 256;  // column groups
+  constexpr int NT = D / 16, NTW = (NT + NCH - 1) / NCH;  // column tiles of a [64 x D] result; a wave's share
   constexpr bool BF = sizeof(TIn) == 2;  // bf16 inputs: the products on bf16 MFMA (fp32 accumulation)
   __shared__ __align__(16) float buf[9][kC * P];
-  __shared__ float sB[kC], sPart[4 * kC], sRow[2 * kC];
+  __shared__ float sB[kC], sPart[4 * kC], sRow[NCH * kC];
   const int c = blockIdx.x % NC, bh = blockIdx.x / NC;
   const int b = bh / H, h = bh - b * H;
   const int t0 = c * kC;
   const size_t chunk = blockIdx.x;
-  const int w = threadIdx.x >> 6, ch = w >> 2, rb = ch == 0 ? w : 7 - w;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ch = w >> 2, rb = (ch & 1) == 0 ? (w & 3) : 3 - (w & 3);
   float *Bq = buf[0], *Bk = buf[1], *Bo = buf[2], *Br = buf[3], *Bh = buf[4], *Bg = buf[5], *Bl = buf[6];
   float *Bd = buf[7], *Bp = buf[8];
   {
@@ -619,13 +625,13 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   __syncthreads();
   const int r0 = 16 * rb;  // this wave's 16 rows of every [64 x .] result
   // R = V - K H, in place (each tile reads only its own V entries)
-  for (int ct = ch; ct < NT; ct += 2) {
+  for (int ct = ch; ct < NT; ct += NCH) {
     const f32x4 acc = mm16<false, false, BF>(Bk + r0 * P, P, Bh + 16 * ct, P, D, zero4());
 #pragma unroll
     for (int r = 0; r < 4; ++r) Br[(r0 + tile_row(r)) * P + 16 * ct + tile_col()] -= acc[r];
   }
   // P = tril(Q K^T), diagonal included (tiles above the diagonal: zeros)
-  for (int ct = ch; ct < 4; ct += 2) {
+  for (int ct = ch; ct < 4; ct += NCH) {
     const f32x4 acc = ct <= rb ? mm16<false, true, BF>(Bq + r0 * P, P, Bk + 16 * ct * P, P, D, zero4()) : zero4();
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -635,7 +641,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   }
   __syncthreads();
   // Delta = L diag(beta) R (L lower triangular: k blocks 0 .. rb)
-  for (int ct = ch; ct < NT; ct += 2) {
+  for (int ct = ch; ct < NT; ct += NCH) {
     const f32x4 acc = mm16k<false, false, BF>(Bl + r0 * P, P, Br + 16 * ct, P, 0, rb + 1, zero4(), sB);
 #pragma unroll
     for (int r = 0; r < 4; ++r) Bd[(r0 + tile_row(r)) * P + 16 * ct + tile_col()] = acc[r];
@@ -647,7 +653,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   f32x4 ddl[NTW];
 #pragma unroll
   for (int u = 0; u < NTW; ++u) {
-    const int ct = ch + 2 * u;
+    const int ct = ch + NCH * u;
     if (ct < NT) {
       ddl[u] = mm16<false, false, BF>(Bk + r0 * P, P, Bg + 16 * ct, P, D, zero4());
       ddl[u] = mm16k<true, false, BF>(Bp + r0, P, Bo + 16 * ct, P, rb, 4, ddl[u]);  // P^T: k blocks rb .. 3
@@ -658,7 +664,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   float* Bdd = Bg;
 #pragma unroll
   for (int u = 0; u < NTW; ++u) {
-    const int ct = ch + 2 * u;
+    const int ct = ch + NCH * u;
     if (ct < NT)
 #pragma unroll
       for (int r = 0; r < 4; ++r) Bdd[(r0 + tile_row(r)) * P + 16 * ct + tile_col()] = ddl[u][r];
@@ -666,7 +672,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   __syncthreads();
   // dR = diag(beta) L^T dDelta into P's buffer (free now); dV = dR
   float* Bdr = Bp;
-  for (int ct = ch; ct < NT; ct += 2) {
+  for (int ct = ch; ct < NT; ct += NCH) {
     const f32x4 acc = mm16k<true, false, BF>(Bl + r0, P, Bdd + 16 * ct, P, rb, 4, zero4());  // L^T: k blocks rb .. 3
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -680,7 +686,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   // dK -= dR H^T
 #pragma unroll
   for (int u = 0; u < NTW; ++u) {
-    const int ct = ch + 2 * u;
+    const int ct = ch + NCH * u;
     if (ct < NT) {
       const f32x4 acc = mm16<false, true, BF>(Bdr + r0 * P, P, Bh + 16 * ct * P, P, D, zero4());
 #pragma unroll
@@ -690,7 +696,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   __syncthreads();  // the reads of dR are done
   // S2 = tril(dO Delta^T), diagonal included, into dR's buffer (tiles above the diagonal: zeros)
   float* Bs = Bp;
-  for (int ct = ch; ct < 4; ct += 2) {
+  for (int ct = ch; ct < 4; ct += NCH) {
     const f32x4 acc = ct <= rb ? mm16<false, true, BF>(Bo + r0 * P, P, Bd + 16 * ct * P, P, D, zero4()) : zero4();
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -702,7 +708,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   // dQ = dO H^T + S2 K; dK += S2^T Q
 #pragma unroll
   for (int u = 0; u < NTW; ++u) {
-    const int ct = ch + 2 * u;
+    const int ct = ch + NCH * u;
     if (ct < NT) {
       f32x4 acc = mm16<false, true, BF>(Bo + r0 * P, P, Bh + 16 * ct * P, P, D, zero4());
       acc = mm16k<false, false, BF>(Bs + r0 * P, P, Bk + 16 * ct, P, 0, rb + 1, acc);  // S2: k blocks 0 .. rb
@@ -718,7 +724,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   // dT = dDelta R^T. dbeta_j gets sum_i dT_ij L_ij (L is zero above its diagonal): each wave sums
   // its 16 rows of its columns into sPart; dL = tril(dT) diag(beta) goes into H's buffer
   float* Bt = Bh;
-  for (int ct = ch; ct < 4; ct += 2) {  // (tiles above the diagonal: dL is zero there, and so is L)
+  for (int ct = ch; ct < 4; ct += NCH) {  // (tiles above the diagonal: dL is zero there, and so is L)
     const f32x4 acc = ct <= rb ? mm16<false, true, BF>(Bdd + r0 * P, P, Br + 16 * ct * P, P, D, zero4()) : zero4();
     const int j = 16 * ct + tile_col();
     float part = 0.f;
@@ -734,7 +740,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   __syncthreads();
   // X1 = L^T dL into Q's buffer (L^T upper, dL lower triangular: k blocks max(rb, ct) .. 3)
   float* Bx = Bq;
-  for (int ct = ch; ct < 4; ct += 2) {
+  for (int ct = ch; ct < 4; ct += NCH) {
     const f32x4 acc = mm16k<true, false, BF>(Bl + r0, P, Bt + 16 * ct, P, max(rb, ct), 4, zero4());
 #pragma unroll
     for (int r = 0; r < 4; ++r) Bx[(r0 + tile_row(r)) * P + 16 * ct + tile_col()] = acc[r];
@@ -744,7 +750,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   // sRow; M = diag(beta) dA goes into dO's buffer
   float* Ba = Bo;
   float rows[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int ct = ch; ct < 4; ct += 2) {
+  for (int ct = ch; ct < 4; ct += NCH) {
     if (ct > rb) {  // strictly above the diagonal: dA and M are zero
 #pragma unroll
       for (int r = 0; r < 4; ++r) Ba[(r0 + tile_row(r)) * P + 16 * ct + tile_col()] = 0.f;
@@ -770,7 +776,7 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   // dK += M K + M^T K, then store
 #pragma unroll
   for (int u = 0; u < NTW; ++u) {
-    const int ct = ch + 2 * u;
+    const int ct = ch + NCH * u;
     if (ct < NT) {
       dka[u] = mm16k<false, false, BF>(Ba + r0 * P, P, Bk + 16 * ct, P, 0, rb + 1, dka[u]);  // M: k blocks 0 .. rb
       dka[u] = mm16k<true, false, BF>(Ba + r0, P, Bk + 16 * ct, P, rb, 4, dka[u]);         // M^T: k blocks rb .. 3
@@ -783,7 +789,10 @@ __global__ __launch_bounds__(kChunkThreads) void scan_bwd_chunk_kernel(
   }
   const int i = threadIdx.x;
   if (i < kC && t0 + i < N) {
-    const float x = ((sPart[i] + sPart[kC + i]) + (sPart[2 * kC + i] + sPart[3 * kC + i])) + (sRow[i] + sRow[kC + i]);
+    float rs = sRow[i];
+#pragma unroll
+    for (int c2 = 1; c2 < NCH; ++c2) rs += sRow[c2 * kC + i];
+    const float x = ((sPart[i] + sPart[kC + i]) + (sPart[2 * kC + i] + sPart[3 * kC + i])) + rs;
     dbeta[((size_t)b * N + t0 + i) * H + h] = from_f32<TIn>(x);
   }
 }
@@ -1668,7 +1677,7 @@ void launch(const TIn* q, const TIn* k, const TIn* v, const TIn* beta, const flo
       hipLaunchKernelGGL((scan_bwd_prep_bf16_kernel<D, false>), dim3(chunks), dim3(kPrepThreads), 0, stream, q, k, v,
                          beta, d_o, active, ws, N, H, NC);
   } else {
-    hipLaunchKernelGGL((scan_bwd_prep_kernel<TIn, D>), dim3(chunks), dim3(kPrepThreads), 0, stream, q, k, v, beta, d_o,
+    hipLaunchKernelGGL((scan_bwd_prep_kernel<TIn, D>), dim3(chunks), dim3(kPrepThreadsF<D>), 0, stream, q, k, v, beta, d_o,
                        active, ws, N, H, NC);
   }
   hipLaunchKernelGGL((scan_bwd_chains_kernel<TIn, D>), dim3(hrec != nullptr ? slices : 2 * slices), dim3(64), 0, stream,
@@ -1681,7 +1690,7 @@ void launch(const TIn* q, const TIn* k, const TIn* v, const TIn* beta, const flo
     hipLaunchKernelGGL((scan_bwd_chunk_bf16_kernel<D>), dim3(chunks), dim3(512), 0, stream, q, k, v, beta, d_o, active,
                        ws, hrec, dq, dk, dv, dbeta, N, H, NC);
   else
-    hipLaunchKernelGGL((scan_bwd_chunk_kernel<TIn, D>), dim3(chunks), dim3(kChunkThreads), 0, stream, q, k, v, beta, d_o,
+    hipLaunchKernelGGL((scan_bwd_chunk_kernel<TIn, D>), dim3(chunks), dim3(kChunkThreads<D>), 0, stream, q, k, v, beta, d_o,
                        active, ws, dq, dk, dv, dbeta, N, H, NC);
 }
 
