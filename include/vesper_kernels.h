@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define VSP_ABI_VERSION 21
+#define VSP_ABI_VERSION 22
 
 /* Status codes. */
 #define VSP_OK 0
@@ -470,6 +470,17 @@ int vsp_halt_step(const uint8_t* active, const uint8_t* exits, int* n_iters, uin
  * as they are. d a multiple of 8; x1, a, x 16-byte aligned; x must not overlap x1 or a. */
 int vsp_residual_rows_where(const float* x1, const void* a, float* x, const uint8_t* flags, int rows, int d,
                             void* stream);
+
+/* The end of a looped column's pass in one launch (vesper/loop.py:441-453, 523-537): over `rows` tokens,
+ * with halts = active & exits (exits NULL: every active token halts, the last pass), n_iters += active
+ * (int32, in place), next = active & !halts, dst[i][r] = src[i][r] for each of `count` (0..8) tensors
+ * where a token halts (as vsp_copy_rows_where), x[r] = x1[r] + a[r] where it was active (as
+ * vsp_residual_rows_where) and norm_out[r] = RMSNorm(x[r]) for every row (bf16, as vsp_rms_norm_bf16
+ * without a gain, bitwise; NULL: none). d a multiple of 8 in 8..2048; x1, a, x, norm_out 16-byte aligned;
+ * x must not overlap x1 or a, nor next be active. */
+int vsp_pass_end(int count, const void* const* src, void* const* dst, const size_t* row_bytes, const float* x1,
+                 const void* a, float* x, const uint8_t* active, const uint8_t* exits, int* n_iters, uint8_t* next,
+                 void* norm_out, int rows, int d, void* stream);
 
 #ifdef __cplusplus
 }

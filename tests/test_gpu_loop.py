@@ -263,3 +263,28 @@ def test_the_residual_rows_match_the_add_and_the_row_copy():
         want = x1 + a if fl is None else torch.where(fl[..., None], x1 + a, x)
         residual_rows_where(x1, a, x, fl)
         assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("d", [8, 512, 520, 1032, 2048])
+@pytest.mark.parametrize(("b", "n"), [(1, 1), (1, 5), (3, 68)])
+@pytest.mark.parametrize(("last", "norm"), [(False, True), (True, False), (False, False)])
+def test_the_pass_end_equals_its_four_launches_bitwise(b, n, d, last, norm):
+    from vesper.kernels.carry import copy_rows_where, end_pass, halt_step, residual_rows_where
+    from vesper.kernels.norm import rms_norm_bf16
+
+    g = torch.Generator().manual_seed(d + n)
+    x1, x = (3 * torch.randn(b, n, d, generator=g).to(GPU) for _ in range(2))
+    a = torch.randn(b, n, d, generator=g).to(GPU, torch.bfloat16)
+    active, exits = (torch.rand(b, n, generator=g).to(GPU) < p for p in (0.7, 0.5))
+    iters = torch.randint(0, 5, (b, n), generator=g, dtype=torch.int32).to(GPU)
+    # rows of 16-, 4- and 2-byte units
+    pairs = [tuple(torch.randn(b, n, *s, generator=g).to(GPU, torch.bfloat16) for _ in range(2)) for s in ((2, 8), (6,), (3,))]
+    ex = None if last else exits
+    want_iters, want_x, want_dst = iters.clone(), x.clone(), [q.clone() for _, q in pairs]
+    halts, want_next = halt_step(active, ex, want_iters)
+    copy_rows_where([(p, q, halts) for (p, _), q in zip(pairs, want_dst)])
+    residual_rows_where(x1, a, want_x, active)
+    nxt, out = end_pass(x1, a, x, active, ex, iters, pairs, norm=norm)
+    assert torch.equal(nxt, want_next) and torch.equal(iters, want_iters) and torch.equal(x, want_x)
+    assert all(torch.equal(q, w) for (_, q), w in zip(pairs, want_dst))
+    assert (out is None) == (not norm) and (out is None or torch.equal(out, rms_norm_bf16(want_x)))

@@ -19,7 +19,7 @@ import torch
 HERE = Path(__file__).resolve().parent
 LIBRARY_PATH = HERE / "libvesper_kernels.so"
 HEADER_PATH = HERE.parents[2] / "include" / "vesper_kernels.h"
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 P = ctypes.c_void_p
 I = ctypes.c_int
@@ -84,6 +84,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "vsp_rms_norm_bf16": (I, [P, P, P, I, I, P]),
     "vsp_add_rms_norm_bf16": (I, [P, P, P, P, P, I, I, P]),
     "vsp_halt_step": (I, [P, P, P, P, P, I, P]),
+    "vsp_pass_end": (I, [I, P, P, P, P, P, P, P, P, P, P, P, I, I, P]),
     "vsp_residual_rows_where": (I, [P, P, P, P, I, I, P]),
     "vsp_delta_step_keys_bf16": (I, [P, P, P, P, P, P, I, P, P, P, P, I, I, I, P]),
     "vsp_decode_proj_bf16": (I, [P, P, P, P, P, I, I, I, I, I, I, I, I, P, P, P, P, I, P, P, I, I, P]),

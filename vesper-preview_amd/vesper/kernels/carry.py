@@ -133,3 +133,57 @@ def residual_rows_where(x1: Tensor, a: Tensor, x: Tensor, flags: Tensor | None) 
     with _lib.on_device(x1.device):
         _lib.call("vsp_residual_rows_where", x1c.data_ptr(), ac.data_ptr(), x.data_ptr(), _lib.ptr(fl), b * n, d,
                   _lib.stream_of(x1.device))
+
+
+def end_pass(x1: Tensor, a: Tensor, x: Tensor, active: Tensor, exits: Tensor | None, n_iters: Tensor,
+             freeze: Sequence[tuple[Tensor, Tensor]], *, norm: bool) -> tuple[Tensor, Tensor | None]:
+    """The end of a looped column's pass in one launch (``vsp_pass_end``): ``halt_step``, then
+    ``copy_rows_where`` of each ``(src, dst)`` of ``freeze`` where a token halts, then
+    ``residual_rows_where(x1, a, x, active)``, then, with ``norm``, ``rms_norm_bf16(x)``; bitwise those
+    launches' results.
+
+    Args:
+        x1: contiguous float32 ``[b, n, d]``; a: contiguous bfloat16 ``[b, n, d]``; x: contiguous
+            float32 ``[b, n, d]``, written in place (not ``x1``); ``d`` a multiple of 8 in 8..2048.
+        active, exits: contiguous bool ``[b, n]`` (``exits`` None: the last pass); n_iters: contiguous
+            int32 ``[b, n]``, counted up in place.
+        freeze: up to eight pairs of contiguous tensors of one shape and dtype, leading ``[b, n]``.
+
+    Returns:
+        the next pass's active flags and its normalized input (None without ``norm``).
+
+    Raises:
+        ContractError: on shapes, dtypes, devices or layouts outside that contract.
+    """
+    lead, device = x1.shape[:2], x1.device
+    if x1.dim() != 3 or x1.dtype != torch.float32 or device.type != "cuda":
+        raise ContractError(f"x1: float32 [b, n, d] on CUDA, got {tuple(x1.shape)} {x1.dtype} on {device}")
+    for name, t, dtype, shape in (("a", a, torch.bfloat16, x1.shape), ("x", x, torch.float32, x1.shape),
+                                  ("active", active, torch.bool, lead), ("n_iters", n_iters, torch.int32, lead),
+                                  ("exits", exits, torch.bool, lead)):
+        if t is not None and (t.dtype != dtype or t.shape != shape or t.device != device):
+            raise ContractError(f"{name}: {dtype} {tuple(shape)} on {device}, got {tuple(t.shape)} {t.dtype} on {t.device}")
+    if len(freeze) > MAX_ITEMS:
+        raise ContractError(f"{len(freeze)} tensors: at most {MAX_ITEMS} per launch")
+    for i, (src, dst) in enumerate(freeze):
+        if src.shape != dst.shape or src.dtype != dst.dtype or src.shape[:2] != lead or src.device != device or dst.device != device:
+            raise ContractError(f"item {i}: src {tuple(src.shape)} {src.dtype}, dst {tuple(dst.shape)} {dst.dtype}")
+    exits_c = None if exits is None else exits.contiguous()
+    if not all(t.is_contiguous() for t in (x1, a, x, active, n_iters, *(t for pair in freeze for t in pair))):
+        raise ContractError("every tensor of a pass's end must be contiguous")
+    if x.data_ptr() == x1.data_ptr():
+        raise ContractError("x must not be x1")
+    b, n, d = x1.shape
+    rows, count = b * n, len(freeze)
+    nxt = torch.empty_like(active)
+    out = torch.empty(b, n, d, dtype=torch.bfloat16, device=device) if norm else None
+    if rows == 0:
+        return nxt, out
+    pointers = ctypes.c_void_p * count
+    srcs, dsts = pointers(*[s.data_ptr() for s, _ in freeze]), pointers(*[t.data_ptr() for _, t in freeze])
+    sizes = (ctypes.c_size_t * count)(*[t.numel() * t.element_size() // rows for _, t in freeze])
+    with _lib.on_device(device):
+        _lib.call("vsp_pass_end", count, ctypes.cast(srcs, ctypes.c_void_p), ctypes.cast(dsts, ctypes.c_void_p),
+                  ctypes.cast(sizes, ctypes.c_void_p), x1.data_ptr(), a.data_ptr(), x.data_ptr(), active.data_ptr(),
+                  _lib.ptr(exits_c), n_iters.data_ptr(), nxt.data_ptr(), _lib.ptr(out), rows, d, _lib.stream_of(device))
+    return nxt, out

@@ -6,48 +6,23 @@
 // whole token rows. Here one launch copies the flagged rows of up to eight tensors in place,
 // dst[r] = src[r] where flags[r] != 0: only the flagged rows are read and written.
 #include "common.h"
+#include "row_items.h"
 #include "vesper_kernels.h"
 
 namespace vsp {
 namespace {
 
-constexpr int kMaxItems = 8;
-
-struct CopyItems {
-  const uint8_t* src[kMaxItems];
-  uint8_t* dst[kMaxItems];
-  const uint8_t* flags[kMaxItems];
-  unsigned row_units[kMaxItems];       // copy units per row
-  unsigned unit_log2[kMaxItems];       // a unit is 1 << unit_log2 bytes (1 .. 16)
-  int count;
+struct RowFlags {
+  const uint8_t* of[kMaxItems];
 };
 
-template <typename U>
-__device__ __forceinline__ void copy_unit(const uint8_t* src, uint8_t* dst, size_t u) {
-  reinterpret_cast<U*>(dst)[u] = reinterpret_cast<const U*>(src)[u];
-}
-
 // One token row per wave, every item in turn: a row whose flag is 0 costs one flag read, a flagged
-// row is copied by the wave's lanes in units of 1 << unit_log2 bytes.
-__global__ __launch_bounds__(256) void copy_rows_kernel(const CopyItems items, unsigned rows) {
-  const unsigned row = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+// row is copied by the wave's lanes.
+__global__ __launch_bounds__(256) void copy_rows_kernel(const RowItems items, const RowFlags flags, unsigned rows) {
+  const unsigned row = blockIdx.x * 4u + (threadIdx.x >> 6);
   if (row >= rows) return;
-  for (int i = 0; i < items.count; ++i) {
-    if (items.flags[i][row] == 0) continue;
-    const unsigned per = items.row_units[i];
-    const size_t base = (size_t)row * per;
-    const uint8_t* s = items.src[i];
-    uint8_t* d = items.dst[i];
-    for (unsigned u = lane; u < per; u += 64) {
-      switch (items.unit_log2[i]) {
-        case 4: copy_unit<uint4>(s, d, base + u); break;
-        case 3: copy_unit<uint2>(s, d, base + u); break;
-        case 2: copy_unit<uint32_t>(s, d, base + u); break;
-        case 1: copy_unit<uint16_t>(s, d, base + u); break;
-        default: copy_unit<uint8_t>(s, d, base + u); break;
-      }
-    }
-  }
+  for (int i = 0; i < items.count; ++i)
+    if (flags.of[i][row] != 0) copy_row_item(items, i, row);
 }
 
 }  // namespace
@@ -61,24 +36,16 @@ extern "C" int vsp_copy_rows_where(int count, const void* const* src, void* cons
   if (rows < 0) return fail(ERR_ARG, "%s: %d rows", who, rows);
   if (count == 0 || rows == 0) return OK;
   if (!src || !dst || !row_bytes || !flags) return fail(ERR_ARG, "%s: null array", who);
-  CopyItems items{};
-  items.count = count;
+  RowItems items{};
+  RowFlags of{};
   for (int i = 0; i < count; ++i) {
-    if (!src[i] || !dst[i] || !flags[i]) return fail(ERR_ARG, "%s: null pointer in tensor %d", who, i);
-    if (row_bytes[i] == 0) return fail(ERR_ARG, "%s: tensor %d has empty rows", who, i);
-    const uintptr_t mix = reinterpret_cast<uintptr_t>(src[i]) | reinterpret_cast<uintptr_t>(dst[i]) | row_bytes[i];
-    unsigned lg = 4;
-    while (lg > 0 && (mix & ((1u << lg) - 1)) != 0) --lg;
-    const size_t per = row_bytes[i] >> lg;
-    if (per > 0xFFFFFFFFu) return fail(ERR_UNSUPPORTED, "%s: rows of %zu bytes", who, row_bytes[i]);
-    items.src[i] = static_cast<const uint8_t*>(src[i]);
-    items.dst[i] = static_cast<uint8_t*>(dst[i]);
-    items.flags[i] = flags[i];
-    items.row_units[i] = (unsigned)per;
-    items.unit_log2[i] = lg;
+    if (!flags[i]) return fail(ERR_ARG, "%s: null pointer in tensor %d", who, i);
+    of.of[i] = flags[i];
   }
+  const int st = row_items(items, count, src, dst, row_bytes, who);
+  if (st != OK) return st;
   hipLaunchKernelGGL(copy_rows_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), items, (unsigned)rows);
+                     reinterpret_cast<hipStream_t>(stream), items, of, (unsigned)rows);
   return check_launch(who);
 }
 

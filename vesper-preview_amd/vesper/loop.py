@@ -21,7 +21,7 @@ The loop zeroes inactive outputs, freezes the projections of tokens as they halt
 into every later pass's state (copy-forward), and carries halted tokens' hidden states forward
 unchanged (``loop.py:441-453``, ``:523-537``). By default (``copy_forward="fused"``) the kernels read
 the carried rows of inactive tokens inside their loads (the key filter's ``carried_z``, the scan's
-``carried``, the attention's ``carried``) and one launch per pass (``copy_rows_where``) freezes the
+``carried``, the attention's ``carried``) and one launch per pass (``end_pass``) freezes the
 halting tokens' projections into the carried buffers and carries the hidden state, in place of the
 reference's ``where`` merges; ``copy_forward="where"`` runs those merges as torch selects.
 
@@ -41,7 +41,7 @@ from torch import Tensor
 from vesper.attention import rotary_qk
 from vesper.column import recurrent_keys
 from vesper.contracts import ContractError, Dims, check_shape
-from vesper.kernels.carry import copy_rows_where, halt_step, residual_rows_where
+from vesper.kernels.carry import end_pass, halt_step, residual_rows_where
 from vesper.kernels.delta_scan import delta_scan_fused
 from vesper.kernels.keys import fused_keys
 from vesper.kernels.norm import projection, rms_norm_bf16
@@ -222,14 +222,13 @@ class LoopedColumn:
         assert history is not None
         return recurrent_keys(z, history, self.taps[t], self.heads, active=active, carried_z=carried_z)
 
-    def _step(self, x: Tensor, t: int, state: Tensor, history: Tensor | None, active: Tensor | None,
+    def _step(self, x: Tensor, xb: Tensor, t: int, state: Tensor, history: Tensor | None, active: Tensor | None,
               carried: Written | None) -> tuple[tuple[Tensor, Tensor], Tensor, Tensor | None, Written]:
-        """One pass over ``x``; returns ``(x1, a)`` (the hidden state after the recurrent sublayer
+        """One pass over ``x`` (``xb``: its norm); returns ``(x1, a)`` (the hidden state after the recurrent sublayer
         and the attention's output: the pass's output is ``x1 + a``), the new state and history, and
         the projections the pass wrote."""
         b, n, d = x.shape
         h, dk = self.heads, self.head_dim
-        xb = rms_norm_bf16(x)
         q_in, z, v, beta = self.project_rec(t, xb)
         q = q_in.view(b, n, h, dk)  # the scan's query is not normalized (column.py:247)
         fused = self.copy_forward == "fused" and carried is not None and active is not None
@@ -297,37 +296,43 @@ class LoopedColumn:
             x = x0
             new_states = list(states)
             new_histories: list[Tensor | None] = list(histories) if histories is not None else [None] * self.passes
+            xb: Tensor | None = None  # the norm of x, where the previous pass's end has written it
             for t in range(self.passes):
+                last = t == self.passes - 1
                 # pass 0 runs with every token active: the unmasked kernels, as the reference's
                 # carry-free first pass
                 mask = None if carried is None else active
-                (x1, a), new_states[t], new_histories[t], written = self._step(x, t, new_states[t],
-                                                                               new_histories[t], mask, carried)
-                # halts = active & exit (all active on the last pass), n_iters += active, and the
-                # next pass's active & ~halts: one launch
-                halts, next_active = halt_step(active, exits[t] if t < self.passes - 1 else None, n_iters)
-                if carried is None:  # pass 0: every token active, the fresh projections are the carried ones
-                    carried = written
-                    x = torch.empty_like(x1)  # this loop's own buffer from here on
-                    residual_rows_where(x1, a, x, None)
-                elif self.copy_forward == "where":
-                    h = x1 + a
-                    h = _where_tokens(active, h, torch.zeros_like(h))
-                    carried = written.merged(halts, carried)
-                    x = _where_tokens(active, h, x)
+                (x1, a), new_states[t], new_histories[t], written = self._step(
+                    x, rms_norm_bf16(x) if xb is None else xb, t, new_states[t], new_histories[t], mask, carried)
+                if self.copy_forward == "where":
+                    # halts = active & exit (all active on the last pass), n_iters += active, and the
+                    # next pass's active & ~halts: one launch
+                    halts, next_active = halt_step(active, None if last else exits[t], n_iters)
+                    if carried is None:
+                        carried = written
+                        x = torch.empty_like(x1)
+                        residual_rows_where(x1, a, x, None)
+                    else:
+                        h = x1 + a
+                        h = _where_tokens(active, h, torch.zeros_like(h))
+                        carried = written.merged(halts, carried)
+                        x = _where_tokens(active, h, x)
                 else:
-                    # one launch: the tokens halting now freeze their fresh projections into the
-                    # carried buffers (none after the last pass); then the active tokens' hidden
-                    # states x1 + a go straight into x (this loop's own buffer from pass 1 on)
-                    items: list[tuple[Tensor, Tensor, Tensor]] = []
-                    if t < self.passes - 1:
-                        items = [(written.k, carried.k, halts), (written.v, carried.v, halts),
-                                 (written.beta, carried.beta, halts), (written.attn_k, carried.attn_k, halts),
-                                 (written.attn_v, carried.attn_v, halts)]
+                    # one launch: the halting bookkeeping, the tokens halting now freezing their fresh
+                    # projections into the carried buffers (on pass 0 the fresh ones are the carried
+                    # ones, and none after the last), the active tokens' hidden states x1 + a straight
+                    # into x (this loop's own buffer from pass 0's end on) and the next pass's norm
+                    freeze: list[tuple[Tensor, Tensor]] = []
+                    if carried is None:
+                        carried = written
+                        x = torch.empty_like(x1)
+                    elif not last:
+                        freeze = [(written.k, carried.k), (written.v, carried.v), (written.beta, carried.beta),
+                                  (written.attn_k, carried.attn_k), (written.attn_v, carried.attn_v)]
                         if written.z is not None and carried.z is not None:
-                            items.append((written.z, carried.z, halts))
-                    copy_rows_where(items)
-                    residual_rows_where(x1, a, x, active)
+                            freeze.append((written.z, carried.z))
+                    next_active, xb = end_pass(x1, a, x, active, None if last else exits[t], n_iters, freeze,
+                                               norm=not last)
                 active = next_active
         hist_out = tuple(t for t in new_histories if t is not None) if self.taps is not None else None
         return LoopResult(y=x, states=tuple(new_states), n_iters=n_iters, histories=hist_out)
