@@ -1439,7 +1439,7 @@ __global__ __launch_bounds__(512, 4) void scan_bwd_chunk_bf16_kernel(
 // The prep kernel on bf16 LDS tiles (bf16 entry, head widths 32, 64 and 128). The UT solve stays
 // in fp32; once it is done its two fp32 buffers hold the bf16 T and P, and (up to D 64) W and U,
 // so that the kernel's LDS (about 74 KB at D 64) lets two workgroups share a CU.
-template <int D, bool REC>
+template <int D>
 __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_bf16_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ k, const __bf16* __restrict__ v,
     const __bf16* __restrict__ beta, const __bf16* __restrict__ d_o, const uint8_t* __restrict__ active,
@@ -1469,12 +1469,12 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_bf16_kernel(
     rk.fetch(k, b, h, t0, N, H);
     rq.fetch(q, b, h, t0, N, H);
     ro.fetch(d_o, b, h, t0, N, H, active);
-    if constexpr (!REC) rv.fetch(v, b, h, t0, N, H);  // V only for U = T V and B = K^T U (the state chain)
+    rv.fetch(v, b, h, t0, N, H);
     rbeta.fetch(beta, b, h, t0, N, H);
     rk.put(sK, LD);
     rq.put(sQ, LD);
     ro.put(sO, LD);
-    if constexpr (!REC) rv.put(sV, LD);
+    rv.put(sV, LD);
     rbeta.put(sB, t0, N);
   }
   __syncthreads();
@@ -1549,7 +1549,7 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_bf16_kernel(
     *reinterpret_cast<bf16x4*>(sT + i * L6 + j) = t;
   }
   __syncthreads();
-  // W = T K and (for the state chain) U = T V over L; P = tril(Q K^T) beside T
+  // W = T K and U = T V over L; P = tril(Q K^T) beside T
   #pragma unroll
   for (int u_ = 0; u_ < NT / 2; ++u_) {
     const int ct = ch + 2 * u_;
@@ -1558,10 +1558,10 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_bf16_kernel(
     for (int kk = 0; kk < kC; kk += 32) {
       const bf16x8 a = frow(sT, L6, r0, kk);
       aw = mma32(a, fcol(sK, LD, 16 * ct, kk), aw);
-      if constexpr (!REC) au = mma32(a, fcol(sV, LD, 16 * ct, kk), au);
+      au = mma32(a, fcol(sV, LD, 16 * ct, kk), au);
     }
     put_tile(sW, LD, r0, 16 * ct, aw);
-    if constexpr (!REC) put_tile(sU, LD, r0, 16 * ct, au);
+    put_tile(sU, LD, r0, 16 * ct, au);
   }
   #pragma unroll
   for (int u_ = 0; u_ < 2; ++u_) {
@@ -1586,8 +1586,7 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_bf16_kernel(
   }
   __syncthreads();
   // the chains' operands, tile (rt, ct) of each [D x D] product: Y = Q^T dO - W^T Z and B = K^T U
-  // in accumulator order, N = -K^T W into NR and N^T = -W^T K into NF (A tile (ct, rt) of each);
-  // with the forward's records (REC) only the reverse chain runs, so B and N^T are not formed
+  // in accumulator order, N = -K^T W into NR and N^T = -W^T K into NF (A tile (ct, rt) of each)
   float* gY = Ws<D>::Y(ws, chunk);
   float* gB = Ws<D>::B(ws, chunk);
   __bf16* gNF = reinterpret_cast<__bf16*>(Ws<D>::NF(ws, chunk));
@@ -1608,8 +1607,8 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_bf16_kernel(
 #pragma unroll
       for (int kk = 0; kk < kC; kk += 32) {
         const bf16x8 ob = fcol(sO, LD, 16 * ct, kk), zb = -fcol(sZ, LD, 16 * ct, kk);
-        const bf16x8 ub = REC ? bf16x8{} : fcol(sU, LD, 16 * ct, kk);
-        const bf16x8 wb = fcol(sW, LD, 16 * ct, kk), kb = REC ? bf16x8{} : fcol(sK, LD, 16 * ct, kk);
+        const bf16x8 ub = fcol(sU, LD, 16 * ct, kk);
+        const bf16x8 wb = fcol(sW, LD, 16 * ct, kk), kb = fcol(sK, LD, 16 * ct, kk);
 #pragma unroll
         for (int j = 0; j < RG; ++j) {
           const int rt = rt0 + RSTEP * (j0 + j);
@@ -1617,10 +1616,8 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_bf16_kernel(
           y[j] = mma32(qa, ob, y[j]);
           y[j] = mma32(wa, zb, y[j]);
           kw[j] = mma32(ka, wb, kw[j]);
-          if constexpr (!REC) {
-            bb[j] = mma32(ka, ub, bb[j]);
-            wk[j] = mma32(wa, kb, wk[j]);
-          }
+          bb[j] = mma32(ka, ub, bb[j]);
+          wk[j] = mma32(wa, kb, wk[j]);
         }
       }
 #pragma unroll
@@ -1636,11 +1633,191 @@ __global__ __launch_bounds__(kPrepThreads) void scan_bwd_prep_bf16_kernel(
         }
         *reinterpret_cast<bf16x4*>(reinterpret_cast<T*>(gY) + accfrag2<NT>(ct, rt, l)) = yb;
         *reinterpret_cast<bf16x4*>(gNR + afrag<NT>(ct, rt, l)) = nr;
-        if constexpr (!REC) {
-          *reinterpret_cast<bf16x4*>(reinterpret_cast<T*>(gB) + accfrag2<NT>(ct, rt, l)) = bbb;
-          *reinterpret_cast<bf16x4*>(gNF + afrag<NT>(ct, rt, l)) = nf;
-        }
+        *reinterpret_cast<bf16x4*>(reinterpret_cast<T*>(gB) + accfrag2<NT>(ct, rt, l)) = bbb;
+        *reinterpret_cast<bf16x4*>(gNF + afrag<NT>(ct, rt, l)) = nf;
       }
+    }
+  }
+}
+
+// The prep kernel where the forward recorded the chunks' starting states (widths 32 and 64): only the
+// reverse chain runs, so V, U, B and N^T are not formed. K and two fp32 buffers are all of its LDS (46
+// KB, three workgroups a CU): A and L, then over A the tiles T (later W) and P (later Z), and over L
+// the tiles Q and dO, held in registers during the solve. Bound by the chain of the solve and its
+// barriers, as the kernel above; with Q, dO and Z in tiles of their own (74 KB, two workgroups a CU) it
+// took 56 us at B16 T1024 H12 d64, this one 46 (33 for its 175 MB at a large copy's rate).
+template <int D>
+__global__ __launch_bounds__(kPrepThreads, 6) void scan_bwd_prep_rec_kernel(
+    const __bf16* __restrict__ q, const __bf16* __restrict__ k, const __bf16* __restrict__ beta,
+    const __bf16* __restrict__ d_o, const uint8_t* __restrict__ active, float* __restrict__ ws, int N, int H, int NC) {
+  using T = __bf16;
+  constexpr int NT = D / 16, NTH = kPrepThreads;
+  constexpr int LD = D + 8, L6 = kC + 8, PF = kC + 8;  // pitches: [64][D] bf16, [64][64] bf16, [64][64] fp32
+  static_assert(2 * kC * L6 * sizeof(T) == kC * PF * sizeof(float) && LD <= L6, "two tiles fit an fp32 buffer");
+  __shared__ __align__(16) T sK[kC * LD];
+  __shared__ __align__(16) float sA[kC * PF], sL[kC * PF];
+  __shared__ float sB[kC];
+  T *const sT = reinterpret_cast<T*>(sA), *const sP = sT + kC * L6, *const sW = sT, *const sZ = sP;
+  T *const sQ = reinterpret_cast<T*>(sL), *const sO = sQ + kC * L6;
+  const int c = blockIdx.x % NC, bh = blockIdx.x / NC;
+  const int b = bh / H, h = bh - b * H;
+  const int t0 = c * kC;
+  const size_t chunk = blockIdx.x;
+  const int w = threadIdx.x >> 6, ch = w >> 2, rb = ch == 0 ? w : 7 - w, r0 = 16 * rb;
+  ChunkRows16<D, NTH> rq, ro;
+  {
+    ChunkRows16<D, NTH> rk;
+    ChunkBeta<T> rbeta;
+    rk.fetch(k, b, h, t0, N, H);
+    rbeta.fetch(beta, b, h, t0, N, H);
+    rq.fetch(q, b, h, t0, N, H);
+    ro.fetch(d_o, b, h, t0, N, H, active);
+    rk.put(sK, LD);
+    rbeta.put(sB, t0, N);
+  }
+  __syncthreads();
+  // A = tril(diag(beta) K K^T, -1) in fp32
+  #pragma unroll
+  for (int u_ = 0; u_ < 2; ++u_) {
+    const int ct = ch + 2 * u_;
+    f32x4 acc = zero4();
+    if (ct <= rb)
+      #pragma unroll
+      for (int kk = 0; kk < D; kk += 32) acc = mma32(frow(sK, LD, r0, kk), frow(sK, LD, 16 * ct, kk), acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = r0 + tile_row(r), j = 16 * ct + tile_col();
+      sA[i * PF + j] = i > j ? sB[i] * acc[r] : 0.f;
+    }
+  }
+  __syncthreads();
+  // L = (I + A)^-1: the diagonal 16x16 blocks by forward substitution (a lane per column of a
+  // block), then L_ij = -L_ii sum_{m = j}^{i - 1} A_im L_mj level by level on fp32 MFMA
+#pragma unroll
+  for (int e = threadIdx.x; e < kC * kC / 4; e += NTH) {
+    const int i = e / (kC / 4), j = 4 * (e % (kC / 4));
+    if (i / 16 < j / 16) *reinterpret_cast<f32x4*>(sL + i * PF + j) = zero4();
+  }
+  if (w == 0) {
+    const int l = threadIdx.x & 63, blk = l >> 4, col = l & 15;
+    const float* ab = sA + 16 * blk * PF + 16 * blk;
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float sum = i == col ? 1.f : 0.f;
+#pragma unroll
+      for (int m = 0; m < i; ++m) sum -= ab[i * PF + m] * x[m];
+      x[i] = sum;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sL[(16 * blk + i) * PF + 16 * blk + col] = x[i];
+  }
+  __syncthreads();
+  #pragma unroll
+  for (int lev = 1; lev < 4; ++lev) {
+    const int i = w + lev, j = w;
+    if (i < 4) {
+      f32x4 y = zero4();
+      #pragma unroll
+      for (int m = j; m < i; ++m)
+        y = mm16<false, false>(sA + 16 * i * PF + 16 * m, PF, sL + 16 * m * PF + 16 * j, PF, 16, y);
+      float* dst = sL + 16 * i * PF + 16 * j;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dst[tile_row(r) * PF + tile_col()] = y[r];
+      wave_sync_lds();
+      const f32x4 x = mm16<false, false>(sL + 16 * i * PF + 16 * i, PF, dst, PF, 16, zero4());
+      wave_sync_lds();
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dst[tile_row(r) * PF + tile_col()] = -x[r];
+    }
+    __syncthreads();
+  }
+  // L into the workspace in bf16 (as the chunk kernel multiplies it); T = L diag(beta) in bf16 over A
+  T* gL = reinterpret_cast<T*>(Ws<D>::L(ws, chunk));
+  for (int e = threadIdx.x; e < kC * kC / 4; e += NTH) {
+    const int i = e / (kC / 4), j = 4 * (e % (kC / 4));
+    const f32x4 x = *reinterpret_cast<const f32x4*>(sL + i * PF + j);
+    bf16x4 lb, t;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      lb[u] = (T)x[u];
+      t[u] = (T)((float)lb[u] * sB[j + u]);
+    }
+    *reinterpret_cast<bf16x4*>(gL + 4 * e) = lb;
+    *reinterpret_cast<bf16x4*>(sT + i * L6 + j) = t;
+  }
+  __syncthreads();
+  // Q and dO over L; W = T K, kept until T has been read
+  rq.put(sQ, LD);
+  ro.put(sO, LD);
+  f32x4 acc[NT / 2];
+#pragma unroll
+  for (int u = 0; u < NT / 2; ++u) {
+    acc[u] = zero4();
+#pragma unroll
+    for (int kk = 0; kk < kC; kk += 32) acc[u] = mma32(frow(sT, L6, r0, kk), fcol(sK, LD, 16 * (ch + 2 * u), kk), acc[u]);
+  }
+  __syncthreads();
+  // W over T; P = tril(Q K^T) beside it
+#pragma unroll
+  for (int u = 0; u < NT / 2; ++u) put_tile(sW, LD, r0, 16 * (ch + 2 * u), acc[u]);
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int ct = ch + 2 * u;
+    f32x4 p = zero4();
+    if (ct <= rb)
+#pragma unroll
+      for (int kk = 0; kk < D; kk += 32) p = mma32(frow(sQ, LD, r0, kk), frow(sK, LD, 16 * ct, kk), p);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] = 16 * ct + tile_col() <= r0 + tile_row(r) ? p[r] : 0.f;
+    put_tile(sP, L6, r0, 16 * ct, p);
+  }
+  __syncthreads();
+  // Z = P^T dO (P^T upper triangular) over P
+#pragma unroll
+  for (int u = 0; u < NT / 2; ++u) {
+    acc[u] = zero4();
+#pragma unroll
+    for (int kk = 0; kk < kC; kk += 32) acc[u] = mma32(fcol(sP, L6, r0, kk), fcol(sO, LD, 16 * (ch + 2 * u), kk), acc[u]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NT / 2; ++u) put_tile(sZ, LD, r0, 16 * (ch + 2 * u), acc[u]);
+  __syncthreads();
+  // the reverse chain's operands, tile (rt, ct) of each [D x D] product: Y = Q^T dO - W^T Z in
+  // accumulator order, N = -K^T W into NR (A tile (ct, rt)); a wave takes row tiles of one column
+  // tile, two at a time where it has two
+  float* gY = Ws<D>::Y(ws, chunk);
+  __bf16* gNR = reinterpret_cast<__bf16*>(Ws<D>::NR(ws, chunk));
+  const int l = threadIdx.x & 63;
+  constexpr int RG = NT * NT >= 16 ? 2 : 1, RSTEP = 8 / NT;  // a wave's row tiles, and the step between them
+  if (w < NT * NT) {
+    const int ct = w % NT, rt0 = w / NT;
+    f32x4 y[RG], kw[RG];
+#pragma unroll
+    for (int j = 0; j < RG; ++j) y[j] = kw[j] = zero4();
+#pragma unroll
+    for (int kk = 0; kk < kC; kk += 32) {
+      const bf16x8 ob = fcol(sO, LD, 16 * ct, kk), zb = -fcol(sZ, LD, 16 * ct, kk), wb = fcol(sW, LD, 16 * ct, kk);
+#pragma unroll
+      for (int j = 0; j < RG; ++j) {
+        const int rt = rt0 + RSTEP * j;
+        y[j] = mma32(fcol(sQ, LD, 16 * rt, kk), ob, y[j]);
+        y[j] = mma32(fcol(sW, LD, 16 * rt, kk), zb, y[j]);
+        kw[j] = mma32(fcol(sK, LD, 16 * rt, kk), wb, kw[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < RG; ++j) {
+      const int rt = rt0 + RSTEP * j;
+      bf16x4 nr, yb;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        nr[r] = (T)(-kw[j][r]);
+        yb[r] = (T)y[j][r];
+      }
+      *reinterpret_cast<bf16x4*>(reinterpret_cast<T*>(gY) + accfrag2<NT>(ct, rt, l)) = yb;
+      *reinterpret_cast<bf16x4*>(gNR + afrag<NT>(ct, rt, l)) = nr;
     }
   }
 }
@@ -1670,12 +1847,16 @@ void launch(const TIn* q, const TIn* k, const TIn* v, const TIn* beta, const flo
   const int NC = (N + kC - 1) / kC;
   const unsigned chunks = (unsigned)((size_t)B * H * NC), slices = (unsigned)((size_t)B * H * (D / 16));
   if constexpr (sizeof(TIn) == 2 && D >= 32) {
-    if (hrec != nullptr)
-      hipLaunchKernelGGL((scan_bwd_prep_bf16_kernel<D, true>), dim3(chunks), dim3(kPrepThreads), 0, stream, q, k, v,
-                         beta, d_o, active, ws, N, H, NC);
-    else
-      hipLaunchKernelGGL((scan_bwd_prep_bf16_kernel<D, false>), dim3(chunks), dim3(kPrepThreads), 0, stream, q, k, v,
-                         beta, d_o, active, ws, N, H, NC);
+    bool recorded = false;
+    if constexpr (D <= 64) {
+      recorded = hrec != nullptr;
+      if (recorded)
+        hipLaunchKernelGGL((scan_bwd_prep_rec_kernel<D>), dim3(chunks), dim3(kPrepThreads), 0, stream, q, k, beta, d_o,
+                           active, ws, N, H, NC);
+    }
+    if (!recorded)
+      hipLaunchKernelGGL((scan_bwd_prep_bf16_kernel<D>), dim3(chunks), dim3(kPrepThreads), 0, stream, q, k, v, beta, d_o,
+                         active, ws, N, H, NC);
   } else {
     hipLaunchKernelGGL((scan_bwd_prep_kernel<TIn, D>), dim3(chunks), dim3(kPrepThreadsF<D>), 0, stream, q, k, v, beta, d_o,
                        active, ws, N, H, NC);
