@@ -463,7 +463,7 @@ def test_bf16_gradients_over_several_chunks_with_an_active_mask(dk):
     _grad_check(delta_scan_fused, _bf16_inputs(2, 300, 3, dk, seed=dk), TOL, active=act)
 
 
-@pytest.mark.parametrize("dk", [32, 64])
+@pytest.mark.parametrize("dk", [16, 32, 64])
 @pytest.mark.parametrize("n", [16, 63, 64, 65, 81, 128])
 def test_bf16_gradients_at_the_edges_of_a_chunk(dk, n):
     # one row block of 16 alone, and a 64-token chunk one under, whole and one over
@@ -520,6 +520,17 @@ def test_fp32_every_gradient_matches_the_oracle_to_float32(b, n, h, dk):
     from vesper.kernels.delta_scan import delta_scan_fused_fp32
 
     _grad_check(delta_scan_fused_fp32, _fp32_inputs(b, n, h, dk), TOL_FP32)
+
+
+@pytest.mark.parametrize("dk", [16, 32, 64])
+@pytest.mark.parametrize("n", [16, 63, 64, 65, 130])
+def test_fp32_gradients_at_the_edges_of_a_chunk(dk, n):
+    # one row block of 16 alone, and a 64-token chunk one under, whole and one over, at each of the
+    # widths' wave counts and buffer overlays
+    from vesper.kernels.delta_scan import delta_scan_fused_fp32
+
+    act = torch.rand(3, n, generator=torch.Generator().manual_seed(n)) < 0.8
+    _grad_check(delta_scan_fused_fp32, _fp32_inputs(3, n, 5, dk), TOL_FP32, active=act)
 
 
 # the shape the reference quotes both fused scans at (kernels/delta_scan.py:22-24, "stage-1 size":

@@ -587,19 +587,25 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
     const TIn* __restrict__ q, const TIn* __restrict__ k, const TIn* __restrict__ v, const TIn* __restrict__ beta,
     const TIn* __restrict__ d_o, const uint8_t* __restrict__ active, const float* __restrict__ ws,
     TIn* __restrict__ dq, TIn* __restrict__ dk, TIn* __restrict__ dv, TIn* __restrict__ dbeta, int N, int H, int NC) {
-  constexpr int P = kPC;  // every buffer is [64][68]
+  // pitches of [64][64] and of [64][D] and [D][D] buffers. At D 64 the late [64][64] matrices lie over the
+  // dead [64][D] ones; below it over P's and over four of them together, so that at D 16 a workgroup
+  // takes 72 KB and two share a CU (nine [64][68] buffers, 158 KB, at every width: float32 and bf16
+  // backward at B32 T2048 H4 d16 246 -> 189 and 209 -> 149 us)
+  constexpr int P = kPC, PD = D + 4, kBuf = kC * PD;
   constexpr int NTH = kChunkThreads<D>, NCH = NTH / 256;  // column groups
   constexpr int NT = D / 16, NTW = (NT + NCH - 1) / NCH;  // column tiles of a [64 x D] result; a wave's share
   constexpr bool BF = sizeof(TIn) == 2;  // bf16 inputs: the products on bf16 MFMA (fp32 accumulation)
-  __shared__ __align__(16) float buf[9][kC * P];
+  __shared__ __align__(16) float buf[7 * kBuf + 2 * kC * P];
+  static_assert(4 * kBuf >= kC * P, "X1 over four dead buffers");
   __shared__ float sB[kC], sPart[4 * kC], sRow[NCH * kC];
   const int c = blockIdx.x % NC, bh = blockIdx.x / NC;
   const int b = bh / H, h = bh - b * H;
   const int t0 = c * kC;
   const size_t chunk = blockIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ch = w >> 2, rb = (ch & 1) == 0 ? (w & 3) : 3 - (w & 3);
-  float *Bq = buf[0], *Bk = buf[1], *Bo = buf[2], *Br = buf[3], *Bh = buf[4], *Bg = buf[5], *Bl = buf[6];
-  float *Bd = buf[7], *Bp = buf[8];
+  float *const Bq = buf, *const Bo = buf + kBuf, *const Bh = buf + 2 * kBuf, *const Bd = buf + 3 * kBuf;
+  float *const Bk = buf + 4 * kBuf, *const Br = buf + 5 * kBuf, *const Bg = buf + 6 * kBuf;
+  float *const Bl = buf + 7 * kBuf, *const Bp = Bl + kC * P;
   {
     ChunkRows<TIn, D, NTH> rq, rk, ro, rv;
     AccRows<D, NTH> mh, mg;
@@ -613,12 +619,12 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
     mg.fetch(Ws<D>::dHs(const_cast<float*>(ws), chunk));
     ml.fetch(Ws<D>::L(const_cast<float*>(ws), chunk));
     rb_.fetch(beta, b, h, t0, N, H);
-    rq.put(Bq, P, t0, N);
-    rk.put(Bk, P, t0, N);
-    ro.put(Bo, P, t0, N);
-    rv.put(Br, P, t0, N);
-    mh.put(Bh, P);
-    mg.put(Bg, P);
+    rq.put(Bq, PD, t0, N);
+    rk.put(Bk, PD, t0, N);
+    ro.put(Bo, PD, t0, N);
+    rv.put(Br, PD, t0, N);
+    mh.put(Bh, PD);
+    mg.put(Bg, PD);
     ml.put(Bl, P);
     rb_.put(sB, t0, N);
   }
@@ -626,13 +632,13 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
   const int r0 = 16 * rb;  // this wave's 16 rows of every [64 x .] result
   // R = V - K H, in place (each tile reads only its own V entries)
   for (int ct = ch; ct < NT; ct += NCH) {
-    const f32x4 acc = mm16<false, false, BF>(Bk + r0 * P, P, Bh + 16 * ct, P, D, zero4());
+    const f32x4 acc = mm16<false, false, BF>(Bk + r0 * PD, PD, Bh + 16 * ct, PD, D, zero4());
 #pragma unroll
-    for (int r = 0; r < 4; ++r) Br[(r0 + tile_row(r)) * P + 16 * ct + tile_col()] -= acc[r];
+    for (int r = 0; r < 4; ++r) Br[(r0 + tile_row(r)) * PD + 16 * ct + tile_col()] -= acc[r];
   }
   // P = tril(Q K^T), diagonal included (tiles above the diagonal: zeros)
   for (int ct = ch; ct < 4; ct += NCH) {
-    const f32x4 acc = ct <= rb ? mm16<false, true, BF>(Bq + r0 * P, P, Bk + 16 * ct * P, P, D, zero4()) : zero4();
+    const f32x4 acc = ct <= rb ? mm16<false, true, BF>(Bq + r0 * PD, PD, Bk + 16 * ct * PD, PD, D, zero4()) : zero4();
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = r0 + tile_row(r), j = 16 * ct + tile_col();
@@ -642,9 +648,9 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
   __syncthreads();
   // Delta = L diag(beta) R (L lower triangular: k blocks 0 .. rb)
   for (int ct = ch; ct < NT; ct += NCH) {
-    const f32x4 acc = mm16k<false, false, BF>(Bl + r0 * P, P, Br + 16 * ct, P, 0, rb + 1, zero4(), sB);
+    const f32x4 acc = mm16k<false, false, BF>(Bl + r0 * P, P, Br + 16 * ct, PD, 0, rb + 1, zero4(), sB);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) Bd[(r0 + tile_row(r)) * P + 16 * ct + tile_col()] = acc[r];
+    for (int r = 0; r < 4; ++r) Bd[(r0 + tile_row(r)) * PD + 16 * ct + tile_col()] = acc[r];
   }
   __syncthreads();
   // dK accumulates in registers: the wave's rows r0, its column tiles ch, ch + 2
@@ -655,9 +661,9 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
   for (int u = 0; u < NTW; ++u) {
     const int ct = ch + NCH * u;
     if (ct < NT) {
-      ddl[u] = mm16<false, false, BF>(Bk + r0 * P, P, Bg + 16 * ct, P, D, zero4());
-      ddl[u] = mm16k<true, false, BF>(Bp + r0, P, Bo + 16 * ct, P, rb, 4, ddl[u]);  // P^T: k blocks rb .. 3
-      dka[u] = mm16<false, true, BF>(Bd + r0 * P, P, Bg + 16 * ct * P, P, D, zero4());
+      ddl[u] = mm16<false, false, BF>(Bk + r0 * PD, PD, Bg + 16 * ct, PD, D, zero4());
+      ddl[u] = mm16k<true, false, BF>(Bp + r0, P, Bo + 16 * ct, PD, rb, 4, ddl[u]);  // P^T: k blocks rb .. 3
+      dka[u] = mm16<false, true, BF>(Bd + r0 * PD, PD, Bg + 16 * ct * PD, PD, D, zero4());
     }
   }
   __syncthreads();  // the reads of G are done: dDelta goes into its buffer
@@ -667,13 +673,13 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
     const int ct = ch + NCH * u;
     if (ct < NT)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) Bdd[(r0 + tile_row(r)) * P + 16 * ct + tile_col()] = ddl[u][r];
+      for (int r = 0; r < 4; ++r) Bdd[(r0 + tile_row(r)) * PD + 16 * ct + tile_col()] = ddl[u][r];
   }
   __syncthreads();
   // dR = diag(beta) L^T dDelta into P's buffer (free now); dV = dR
   float* Bdr = Bp;
   for (int ct = ch; ct < NT; ct += NCH) {
-    const f32x4 acc = mm16k<true, false, BF>(Bl + r0, P, Bdd + 16 * ct, P, rb, 4, zero4());  // L^T: k blocks rb .. 3
+    const f32x4 acc = mm16k<true, false, BF>(Bl + r0, P, Bdd + 16 * ct, PD, rb, 4, zero4());  // L^T: k blocks rb .. 3
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = r0 + tile_row(r), j = 16 * ct + tile_col();
@@ -688,7 +694,7 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
   for (int u = 0; u < NTW; ++u) {
     const int ct = ch + NCH * u;
     if (ct < NT) {
-      const f32x4 acc = mm16<false, true, BF>(Bdr + r0 * P, P, Bh + 16 * ct * P, P, D, zero4());
+      const f32x4 acc = mm16<false, true, BF>(Bdr + r0 * P, P, Bh + 16 * ct * PD, PD, D, zero4());
 #pragma unroll
       for (int r = 0; r < 4; ++r) dka[u][r] -= acc[r];
     }
@@ -697,7 +703,7 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
   // S2 = tril(dO Delta^T), diagonal included, into dR's buffer (tiles above the diagonal: zeros)
   float* Bs = Bp;
   for (int ct = ch; ct < 4; ct += NCH) {
-    const f32x4 acc = ct <= rb ? mm16<false, true, BF>(Bo + r0 * P, P, Bd + 16 * ct * P, P, D, zero4()) : zero4();
+    const f32x4 acc = ct <= rb ? mm16<false, true, BF>(Bo + r0 * PD, PD, Bd + 16 * ct * PD, PD, D, zero4()) : zero4();
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = r0 + tile_row(r), j = 16 * ct + tile_col();
@@ -710,22 +716,22 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
   for (int u = 0; u < NTW; ++u) {
     const int ct = ch + NCH * u;
     if (ct < NT) {
-      f32x4 acc = mm16<false, true, BF>(Bo + r0 * P, P, Bh + 16 * ct * P, P, D, zero4());
-      acc = mm16k<false, false, BF>(Bs + r0 * P, P, Bk + 16 * ct, P, 0, rb + 1, acc);  // S2: k blocks 0 .. rb
+      f32x4 acc = mm16<false, true, BF>(Bo + r0 * PD, PD, Bh + 16 * ct * PD, PD, D, zero4());
+      acc = mm16k<false, false, BF>(Bs + r0 * P, P, Bk + 16 * ct, PD, 0, rb + 1, acc);  // S2: k blocks 0 .. rb
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int i = r0 + tile_row(r), j = 16 * ct + tile_col();
         if (t0 + i < N) dq[(((size_t)b * N + t0 + i) * H + h) * D + j] = from_f32<TIn>(acc[r]);
       }
-      dka[u] = mm16k<true, false, BF>(Bs + r0, P, Bq + 16 * ct, P, rb, 4, dka[u]);  // S2^T: k blocks rb .. 3
+      dka[u] = mm16k<true, false, BF>(Bs + r0, P, Bq + 16 * ct, PD, rb, 4, dka[u]);  // S2^T: k blocks rb .. 3
     }
   }
   __syncthreads();  // H, dO, Q, S2, Delta are done with
   // dT = dDelta R^T. dbeta_j gets sum_i dT_ij L_ij (L is zero above its diagonal): each wave sums
   // its 16 rows of its columns into sPart; dL = tril(dT) diag(beta) goes into H's buffer
-  float* Bt = Bh;
+  float* Bt = D == 64 ? Bh : Bp;
   for (int ct = ch; ct < 4; ct += NCH) {  // (tiles above the diagonal: dL is zero there, and so is L)
-    const f32x4 acc = ct <= rb ? mm16<false, true, BF>(Bdd + r0 * P, P, Br + 16 * ct * P, P, D, zero4()) : zero4();
+    const f32x4 acc = ct <= rb ? mm16<false, true, BF>(Bdd + r0 * PD, PD, Br + 16 * ct * PD, PD, D, zero4()) : zero4();
     const int j = 16 * ct + tile_col();
     float part = 0.f;
 #pragma unroll
@@ -739,7 +745,7 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
   }
   __syncthreads();
   // X1 = L^T dL into Q's buffer (L^T upper, dL lower triangular: k blocks max(rb, ct) .. 3)
-  float* Bx = Bq;
+  float* Bx = Bq;  // (below D 64 over Q, dO, H and Delta)
   for (int ct = ch; ct < 4; ct += NCH) {
     const f32x4 acc = mm16k<true, false, BF>(Bl + r0, P, Bt + 16 * ct, P, max(rb, ct), 4, zero4());
 #pragma unroll
@@ -748,7 +754,7 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
   __syncthreads();
   // dA = -tril(X1 L^T, -1); dbeta_i gets sum_{m < i} dA_im (k_i . k_m), each wave's columns into
   // sRow; M = diag(beta) dA goes into dO's buffer
-  float* Ba = Bo;
+  float* Ba = D == 64 ? Bo : Bp;
   float rows[4] = {0.f, 0.f, 0.f, 0.f};
   for (int ct = ch; ct < 4; ct += NCH) {
     if (ct > rb) {  // strictly above the diagonal: dA and M are zero
@@ -758,7 +764,7 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
     }
     // L^T column block ct: k blocks 0 .. ct
     const f32x4 acc = mm16k<false, true, BF>(Bx + r0 * P, P, Bl + 16 * ct * P, P, 0, ct + 1, zero4());
-    const f32x4 gk = mm16<false, true, BF>(Bk + r0 * P, P, Bk + 16 * ct * P, P, D, zero4());
+    const f32x4 gk = mm16<false, true, BF>(Bk + r0 * PD, PD, Bk + 16 * ct * PD, PD, D, zero4());
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = r0 + tile_row(r), j = 16 * ct + tile_col();
@@ -778,8 +784,8 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
   for (int u = 0; u < NTW; ++u) {
     const int ct = ch + NCH * u;
     if (ct < NT) {
-      dka[u] = mm16k<false, false, BF>(Ba + r0 * P, P, Bk + 16 * ct, P, 0, rb + 1, dka[u]);  // M: k blocks 0 .. rb
-      dka[u] = mm16k<true, false, BF>(Ba + r0, P, Bk + 16 * ct, P, rb, 4, dka[u]);         // M^T: k blocks rb .. 3
+      dka[u] = mm16k<false, false, BF>(Ba + r0 * P, P, Bk + 16 * ct, PD, 0, rb + 1, dka[u]);  // M: k blocks 0 .. rb
+      dka[u] = mm16k<true, false, BF>(Ba + r0, P, Bk + 16 * ct, PD, rb, 4, dka[u]);         // M^T: k blocks rb .. 3
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int i = r0 + tile_row(r), j = 16 * ct + tile_col();
