@@ -36,10 +36,12 @@ constexpr float kLazy = 8.f;
 //  * kSrcCached: rows below M from keys / values as the cache alone ([B, M, HKV, D]) and rows M + t
 //    from keys_c / values_c row t (the chunk's own keys and values, [B, N, HKV, D]), so a chunk
 //    attends over a cache without the two being copied into one tensor first. Whole tiles on either
-//    side go through a buffer resource over their tensor; the one tile across row M picks each
-//    row's source by a per-lane address.
-// The per-lane 64-bit source addresses need more registers: three workgroups per CU at D 64
-// instead of four.
+//    side go through a buffer resource over their tensor; the one tile across row M takes each
+//    row from its own.
+// A tile of both sources loads in two turns under the execution mask, one a resource (per-lane 64-bit
+// addresses instead cost registers the whole kernel paid for: 336 / 2048 workgroups cached 25.7 / 80.2 us
+// against 22.7 / 71.6, plain 21.6 / 65.5). Three workgroups per CU at D 64 instead of four: within 128
+// registers both variants spill 49 (29 and 45 us at 336).
 constexpr int kSrcPlain = 0, kSrcCarried = 1, kSrcCached = 2;
 template <typename T, int D, int SRC>
 __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPlain && D == 64 ? 3 : 4))) void window_attn_kernel(const T* __restrict__ q, const T* __restrict__ keys,
@@ -158,8 +160,8 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPla
       CACHED ? (M > 0 ? (unsigned)(((size_t)(M - 1) * kv_row + D) * sizeof(T)) : 0u)
              : (unsigned)(((size_t)(S - 1) * kv_row + D) * sizeof(T));
   const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(kbase, kv_bytes), rv = buffer_rsrc(vbase, kv_bytes);
-  // cached: the chunk's rows, from key index M on
-  const unsigned kvc_bytes = CACHED ? (unsigned)(((size_t)(N - 1) * kv_row + D) * sizeof(T)) : 0u;
+  // cached: the chunk's rows, from key index M on; carried: the carried ones
+  const unsigned kvc_bytes = CACHED || CARRY ? (unsigned)(((size_t)(N - 1) * kv_row + D) * sizeof(T)) : 0u;
   const __amdgpu_buffer_rsrc_t rkc = buffer_rsrc(kcbase + (size_t)M * kv_row, kvc_bytes);
   const __amdgpu_buffer_rsrc_t rvc = buffer_rsrc(vcbase + (size_t)M * kv_row, kvc_bytes);
   unsigned koff[kDirect ? NI : 1], voff[kDirect ? NI : 1];
@@ -188,18 +190,20 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPla
         }
       }
       if constexpr (kDirect && (CARRY || CACHED)) {
-        // per-lane sources (global direct loads: a buffer resource cannot differ between lanes);
-        // rows past the last key re-read key S - 1, from that key's own source (masked in the
-        // scores, they must still be finite: probability 0 times the row)
+        // Per-lane sources: a buffer resource is one for the wave, so the lanes of each source load
+        // in turn under the execution mask (a direct load writes a lane's 16 bytes to the lane's own
+        // place, whichever lanes take part). Rows past the last key read zeros, as plainly loaded
+        // ones (masked in the scores: probability 0 times a finite row).
         const int ins = w + 4 * j;
-        const int pos = ins * 64 + l;
-        const int row = pos / PSEG, seg = pos - row * PSEG;
-        const int rowv = pos / PSEGV, segv = pos - rowv * PSEGV;
-        const int key = min(k0 + row, S - 1), keyv = min(k0 + rowv, S - 1);
-        const size_t sk = (size_t)key * kv_row + 8 * (seg < SEG ? seg ^ kswz(row) : 0);
-        const size_t sv = (size_t)keyv * kv_row + 8 * (segv < SEG ? segv : 0);
-        if (ins < NINS) load_lds16((((fresh >> (key - k0)) & 1) ? kbase : kcbase) + sk, Kn + ins * 64 * 8);
-        if (ins < NINSV) load_lds16((((fresh >> (keyv - k0)) & 1) ? vbase : vcbase) + sv, Vn + ins * 64 * 8);
+        const unsigned toff = (unsigned)((size_t)k0 * kv_row * sizeof(T)), moff = (unsigned)((size_t)M * kv_row * sizeof(T));
+        if (ins < NINS) {
+          if ((fresh >> ((ins * 64 + l) / PSEG)) & 1) buffer_load_lds16(rk, Kn + ins * 64 * 8, koff[j] + toff, 0);
+          else buffer_load_lds16(rkc, Kn + ins * 64 * 8, koff[j] + toff - moff, 0);
+        }
+        if (ins < NINSV) {
+          if ((fresh >> ((ins * 64 + l) / PSEGV)) & 1) buffer_load_lds16(rv, Vn + ins * 64 * 8, voff[j] + toff, 0);
+          else buffer_load_lds16(rvc, Vn + ins * 64 * 8, voff[j] + toff - moff, 0);
+        }
       } else if constexpr (kDirect) {
         const int ins = w + 4 * j;  // this wave's j-th instruction of the tile
         const unsigned toff = (unsigned)((size_t)k0 * kv_row * sizeof(T));
