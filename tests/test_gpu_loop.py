@@ -288,3 +288,27 @@ def test_the_pass_end_equals_its_four_launches_bitwise(b, n, d, last, norm):
     assert torch.equal(nxt, want_next) and torch.equal(iters, want_iters) and torch.equal(x, want_x)
     assert all(torch.equal(q, w) for (_, q), w in zip(pairs, want_dst))
     assert (out is None) == (not norm) and (out is None or torch.equal(out, rms_norm_bf16(want_x)))
+
+
+def test_the_pass_end_takes_strided_sources():
+    from vesper.contracts import ContractError
+    from vesper.kernels.carry import end_pass
+
+    g = torch.Generator().manual_seed(3)
+    b, n, d = 2, 37, 64
+    x1, x = (torch.randn(b, n, d, generator=g).to(GPU) for _ in range(2))
+    a = torch.randn(b, n, d, generator=g).to(GPU, torch.bfloat16)
+    active, exits = (torch.rand(b, n, generator=g).to(GPU) < p for p in (0.7, 0.5))
+    src, dst = (torch.randn(b, n, 4, 8, generator=g).to(GPU, torch.bfloat16) for _ in range(2))
+
+    def strided(t):  # the same values, every other element of the last axis
+        return torch.stack((t, t), dim=-1)[..., 0]
+
+    results = []
+    for wrap in (lambda t: t, strided):
+        xs, ds, iters = x.clone(), dst.clone(), torch.zeros(b, n, dtype=torch.int32, device=GPU)
+        nxt, out = end_pass(wrap(x1), wrap(a), xs, wrap(active), wrap(exits), iters, [(wrap(src), ds)], norm=True)
+        results.append((xs, ds, iters, nxt, out))
+    assert all(torch.equal(p, q) for p, q in zip(*results))
+    with pytest.raises(ContractError):
+        end_pass(x1, a, x, active, exits, torch.zeros(b, n, dtype=torch.int32, device=GPU), [(src, strided(dst))], norm=True)

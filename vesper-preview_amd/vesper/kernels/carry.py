@@ -143,11 +143,12 @@ def end_pass(x1: Tensor, a: Tensor, x: Tensor, active: Tensor, exits: Tensor | N
     launches' results.
 
     Args:
-        x1: contiguous float32 ``[b, n, d]``; a: contiguous bfloat16 ``[b, n, d]``; x: contiguous
-            float32 ``[b, n, d]``, written in place (not ``x1``); ``d`` a multiple of 8 in 8..2048.
-        active, exits: contiguous bool ``[b, n]`` (``exits`` None: the last pass); n_iters: contiguous
-            int32 ``[b, n]``, counted up in place.
-        freeze: up to eight pairs of contiguous tensors of one shape and dtype, leading ``[b, n]``.
+        x1: float32 ``[b, n, d]``; a: bfloat16 ``[b, n, d]``; x: contiguous float32 ``[b, n, d]``,
+            written in place (not ``x1``); ``d`` a multiple of 8 in 8..2048.
+        active, exits: bool ``[b, n]`` (``exits`` None: the last pass); n_iters: contiguous int32
+            ``[b, n]``, counted up in place.
+        freeze: up to eight pairs of one shape and dtype, leading ``[b, n]``, the second contiguous
+            (written in place).
 
     Returns:
         the next pass's active flags and its normalized input (None without ``norm``).
@@ -168,9 +169,11 @@ def end_pass(x1: Tensor, a: Tensor, x: Tensor, active: Tensor, exits: Tensor | N
     for i, (src, dst) in enumerate(freeze):
         if src.shape != dst.shape or src.dtype != dst.dtype or src.shape[:2] != lead or src.device != device or dst.device != device:
             raise ContractError(f"item {i}: src {tuple(src.shape)} {src.dtype}, dst {tuple(dst.shape)} {dst.dtype}")
+    if not all(t.is_contiguous() for t in (x, n_iters, *(dst for _, dst in freeze))):
+        raise ContractError("x, n_iters and every freeze target must be contiguous (they are written in place)")
+    x1, a, active = x1.contiguous(), a.contiguous(), active.contiguous()
     exits_c = None if exits is None else exits.contiguous()
-    if not all(t.is_contiguous() for t in (x1, a, x, active, n_iters, *(t for pair in freeze for t in pair))):
-        raise ContractError("every tensor of a pass's end must be contiguous")
+    sources = [src.contiguous() for src, _ in freeze]
     if x.data_ptr() == x1.data_ptr():
         raise ContractError("x must not be x1")
     b, n, d = x1.shape
@@ -180,7 +183,7 @@ def end_pass(x1: Tensor, a: Tensor, x: Tensor, active: Tensor, exits: Tensor | N
     if rows == 0:
         return nxt, out
     pointers = ctypes.c_void_p * count
-    srcs, dsts = pointers(*[s.data_ptr() for s, _ in freeze]), pointers(*[t.data_ptr() for _, t in freeze])
+    srcs, dsts = pointers(*[s.data_ptr() for s in sources]), pointers(*[t.data_ptr() for _, t in freeze])
     sizes = (ctypes.c_size_t * count)(*[t.numel() * t.element_size() // rows for _, t in freeze])
     with _lib.on_device(device):
         _lib.call("vsp_pass_end", count, ctypes.cast(srcs, ctypes.c_void_p), ctypes.cast(dsts, ctypes.c_void_p),

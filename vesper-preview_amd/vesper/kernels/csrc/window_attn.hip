@@ -193,16 +193,19 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPla
         // Per-lane sources: a buffer resource is one for the wave, so the lanes of each source load
         // in turn under the execution mask (a direct load writes a lane's 16 bytes to the lane's own
         // place, whichever lanes take part). Rows past the last key read zeros, as plainly loaded
-        // ones (masked in the scores: probability 0 times a finite row).
+        // ones (masked in the scores: probability 0 times a finite row); their offsets saturate, since
+        // a batch row of almost 4 GiB would wrap them to its first rows.
         const int ins = w + 4 * j;
         const unsigned toff = (unsigned)((size_t)k0 * kv_row * sizeof(T)), moff = (unsigned)((size_t)M * kv_row * sizeof(T));
         if (ins < NINS) {
-          if ((fresh >> ((ins * 64 + l) / PSEG)) & 1) buffer_load_lds16(rk, Kn + ins * 64 * 8, koff[j] + toff, 0);
-          else buffer_load_lds16(rkc, Kn + ins * 64 * 8, koff[j] + toff - moff, 0);
+          const unsigned at = __builtin_elementwise_add_sat(koff[j], toff);
+          if ((fresh >> ((ins * 64 + l) / PSEG)) & 1) buffer_load_lds16(rk, Kn + ins * 64 * 8, at, 0);
+          else buffer_load_lds16(rkc, Kn + ins * 64 * 8, at - moff, 0);
         }
         if (ins < NINSV) {
-          if ((fresh >> ((ins * 64 + l) / PSEGV)) & 1) buffer_load_lds16(rv, Vn + ins * 64 * 8, voff[j] + toff, 0);
-          else buffer_load_lds16(rvc, Vn + ins * 64 * 8, voff[j] + toff - moff, 0);
+          const unsigned at = __builtin_elementwise_add_sat(voff[j], toff);
+          if ((fresh >> ((ins * 64 + l) / PSEGV)) & 1) buffer_load_lds16(rv, Vn + ins * 64 * 8, at, 0);
+          else buffer_load_lds16(rvc, Vn + ins * 64 * 8, at - moff, 0);
         }
       } else if constexpr (kDirect) {
         const int ins = w + 4 * j;  // this wave's j-th instruction of the tile
