@@ -19,10 +19,13 @@
 //   and Q^T fragments from transposed LDS reads.
 // Both launch 8 waves a workgroup: a staged tile then serves 128 queries (keys), against 64 at 4
 // waves, which cuts the window's overlap re-fetch about in half (dq 69.7 -> 62.0 us, dkv 97.2 ->
-// 86.5 us at B4 T4096 H8 d64 w512); 16 waves measured slower for both.
+// 86.5 us at B4 T4096 H8 d64 w512); 16 waves measured slower for both. Where that leaves the dK/dV
+// kernel with few workgroups, it runs 4 waves (launch_backward).
 #include "attn_mma.h"
 #include "common.h"
 #include "vesper_kernels.h"
+
+#include <type_traits>
 
 namespace vsp {
 namespace {
@@ -238,9 +241,26 @@ __global__ __launch_bounds__(64 * NW, WAVES_PER_SIMD) void attn_dkv_kernel(const
   __shared__ __align__(16) T sQ[2][64 * Sh::P];
   __shared__ __align__(16) T sD[2][64 * Sh::P];
   __shared__ __align__(16) float sL[2][64], sS[2][64];
-  // consecutive key tiles of a KV head on one XCD: their query ranges overlap (L2 hits for Q, dO)
+  // a KV head's key tiles on one XCD: their query ranges overlap (L2 hits for Q, dO)
   const int lg = xcd_logical_block(blockIdx.x, gridDim.x);
-  const int kt = lg % nkt, bkv = lg / nkt;
+  int kt = lg % nkt, bkv = lg / nkt;
+  if constexpr (NW < 8) {
+    // The tiles seen by the most queries first: keys from M to S - W are seen by W queries each, those
+    // before and after by fewer, so the tiles go outward from the middle of that range, and the XCD's
+    // heads take turns. With a head's tiles in order instead the heavy tiles of two heads met on one
+    // CU while others held light ones (at B16 N1024 M512 H8 over 2: 111 against 106 us a backward).
+    const int heads = (int)gridDim.x / nkt;
+    int rank = kt;
+    if (heads % 8 == 0) {
+      const int per = heads >> 3, r = (int)blockIdx.x >> 3;
+      rank = r / per;
+      bkv = (int)(blockIdx.x & 7) * per + (r - rank * per);
+    }
+    const int mid = min((int)(((unsigned)M + (unsigned)max(M + N - W, 0)) / 2u / (16u * NW * KB)), nkt - 1);
+    const int both = min(mid, nkt - 1 - mid);  // tiles on each side before one side ends
+    if (rank <= 2 * both) kt = mid + ((rank & 1) ? -((rank + 1) >> 1) : rank >> 1);
+    else kt = mid > both ? mid - (rank - both) : mid + (rank - both);
+  }
   const int b = bkv / HKV, kvh = bkv - b * HKV;
   const int G = H / HKV;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -403,17 +423,30 @@ void launch_backward(const T* q, const T* keys, const T* values, const T* o, con
   // waves a workgroup (16 queries a dQ wave, 16 KB keys a dK/dV wave); the dK/dV kernel's bound
   // asks for 2 waves a SIMD at least (256 VGPRs): its D 64 instance takes 126 and so runs 4 (two
   // workgroups a CU). Two key blocks a wave (each Q, dO fragment feeding two MFMAs) took 202
-  // VGPRs, halving that, and ran slower (dK/dV 67 -> 77 us at B4 T4096 H8 d64 w512).
+  // VGPRs, halving that, and ran slower (dK/dV 67 -> 77 us at B4 T4096 H8 d64 w512); two query blocks
+  // a dQ wave (168 VGPRs, three waves a SIMD) too (a backward 103 -> 113 us there).
   constexpr int kDqWaves = 8, kDkvWaves = 8, kDkvWavesPerSimd = 2, kDkvBlocks = 1;
   const int nqt = (N + 16 * kDqWaves - 1) / (16 * kDqWaves);
   const int nkt = (M + N + 16 * kDkvWaves * kDkvBlocks - 1) / (16 * kDkvWaves * kDkvBlocks);
   hipLaunchKernelGGL((attn_dq_kernel<T, D, kDqWaves>), dim3((unsigned)((size_t)nqt * H * B)), dim3(64 * kDqWaves), 0,
                      stream, q, keys,
                      values, o, dout, lse, dsum, dq, N, M, H, HKV, W, scale, scale_log2, nqt);
-  hipLaunchKernelGGL((attn_dkv_kernel<T, D, kDkvWaves, kDkvWavesPerSimd, kDkvBlocks>),
-                     dim3((unsigned)((size_t)nkt * HKV * B)),
-                     dim3(64 * kDkvWaves), 0, stream, q, keys,
-                     values, dout, lse, dsum, dk, dv, N, M, H, HKV, W, scale, scale_log2, nkt);
+  auto dkv = [&](auto waves, int tiles) {
+    hipLaunchKernelGGL((attn_dkv_kernel<T, D, decltype(waves)::value, kDkvWavesPerSimd, kDkvBlocks>),
+                       dim3((unsigned)((size_t)tiles * HKV * B)), dim3(64 * decltype(waves)::value), 0, stream, q, keys,
+                       values, dout, lse, dsum, dk, dv, N, M, H, HKV, W, scale, scale_log2, tiles);
+  };
+  // Up to three 8-wave workgroups a CU, a workgroup's chain of steps (the group's heads times its query
+  // tiles, one after the other) and the CUs' unequal shares set the time: half the keys a workgroup make
+  // the chain shorter and the shares more even. Beyond, the tiles' staging counts for more. A whole
+  // backward, 8 / 4 waves, us: B16 N1024 M512 H8 over 2 (384 workgroups) 128.9 / 106.1, B8 N1024 H8 over
+  // 2 (128) 86.4 / 75.8, B3 N4096 H6 (576) 83.7 / 76.4, B8 N1024 M512 H8 (768) 69.8 / 59.1, B4 N4096 H8
+  // (1024) 103.1 / 105.7, B8 N2048 H8 (1024) 102.0 / 104.9. Wider heads fill the LDS with two workgroups
+  // of either size.
+  if (D <= 64 && (size_t)nkt * HKV * B <= 768)
+    dkv(std::integral_constant<int, kDkvWaves / 2>{}, (M + N + 16 * kDkvWaves / 2 - 1) / (16 * kDkvWaves / 2));
+  else
+    dkv(std::integral_constant<int, kDkvWaves>{}, nkt);
 }
 
 template <typename T>
