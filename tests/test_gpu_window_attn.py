@@ -287,6 +287,21 @@ def test_the_reference_benchmark_shape_b16_n1024_m512_h8_hkv2_d64():
         assert relative_error(a, b) < 1e-2, (name, relative_error(a, b))
 
 
+# either side of each line of the launches: dK/dV in 4-wave workgroups up to 768 8-wave ones (48 batch rows
+# of 8 KV heads, two and three 128-key tiles; 97 over one), its heads a multiple of 8 or not; the query
+# tiles heavy first (512 workgroups or more, a quarter of the tiles before the window is full) or in order
+@pytest.mark.parametrize(("b", "n", "m", "w", "h", "hkv"), [
+    (48, 200, 56, 64, 8, 8), (48, 200, 57, 64, 8, 8), (97, 1000, 24, 100, 1, 1), (3, 200, 40, 64, 6, 3),
+    (8, 1000, 0, 512, 8, 2), (8, 897, 300, 512, 8, 4), (8, 1000, 500, 512, 8, 2), (9, 1025, 0, 129, 7, 7)])
+def test_the_gradients_on_either_side_of_the_launch_rules(b, n, m, w, h, hkv):
+    q, keys, values = _inputs(b, n, m, h, hkv, 64, seed=n + m)
+    up = torch.randn(b, n, h, 64, generator=torch.Generator().manual_seed(n)).to(BF16)
+    got = _grads(q, keys, values, w, up)
+    want = _oracle_grads(q, keys, values, w, up, dtype=torch.float32)
+    for a, x, name in zip(got, want, ("o", "dq", "dk", "dv")):
+        assert relative_error(a, x) < 1e-2, name
+
+
 def test_captured_forward_and_backward_equal_eager():
     from vesper.kernels.window_attn import window_attention
 

@@ -39,5 +39,27 @@ __device__ __forceinline__ float max_over_groups(float x) {
   return fmax_ieee(__uint_as_float(c[0]), __uint_as_float(c[1]));
 }
 
+// The workgroup's query tile (of nqt of QT queries) and (batch, head) of a kernel that walks each
+// query's window of W keys. A head's tiles run on one XCD, in order: their key windows overlap, so most
+// of each tile's K and V reads hit that XCD's L2. The first tiles see fewer than W keys. Where they are
+// a quarter of a head's tiles or more and a CU holds two workgroups or more, in that order some CUs get
+// several heavy tiles and others light ones; there the heavy tiles go first, the XCD's heads taking
+// turns (plain attention, in order / heavy first, us: B16 N1024 H8 30.2 / 27.1, B8 N1024 H8 over 2 20.2 /
+// 18.7, B9 N1024 M300 H8 24.8 / 21.8, B8 N2048 H8 31.4 / 30.4). Longer sequences keep the order, whose
+// K and V reuse counts for more there (B4 N4096 H8 31.5 / 33.2).
+__device__ __forceinline__ void query_tile(int nqt, int M, int N, int W, int QT, int& qt, int& bh) {
+  const int heads = (int)gridDim.x / nqt;
+  const int light = (max(min(W, M + N) - 1 - M, 0) + QT - 1) / QT;
+  if (heads % 8 == 0 && gridDim.x >= 512 && 4 * light >= nqt) {
+    const int per = heads >> 3, r = (int)blockIdx.x >> 3, rank = r / per;
+    bh = (int)(blockIdx.x & 7) * per + (r - rank * per);
+    qt = nqt - 1 - rank;
+  } else {
+    const int lg = xcd_logical_block(blockIdx.x, gridDim.x);
+    bh = lg / nqt;
+    qt = lg - bh * nqt;
+  }
+}
+
 }  // namespace
 }  // namespace vsp

@@ -82,8 +82,8 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPla
   __shared__ __align__(16) T sV0[KT * PV], sV1[KT * PV];
 
   auto kswz = [](int row) { return kSwzK ? 2 * ((row >> 1) & 3) : 0; };  // K's segment swizzle
-  const int lg = xcd_logical_block(blockIdx.x, gridDim.x);
-  const int qt = lg % nqt, bh = lg / nqt;
+  int qt, bh;
+  query_tile(nqt, M, N, W, QT, qt, bh);
   const int b = bh / H, h = bh - b * H;
   const int kvh = h / (H / HKV);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;

@@ -103,10 +103,8 @@ __global__ __launch_bounds__(64 * NW) void attn_dq_kernel(const T* __restrict__ 
   constexpr int KT = 64;
   __shared__ __align__(16) T sK[2][KT * Sh::P];
   __shared__ __align__(16) T sV[2][KT * Sh::P];
-  // consecutive query tiles of a head on one XCD: their key windows overlap, so most of each
-  // tile's K and V reads hit that XCD's L2
-  const int lg = xcd_logical_block(blockIdx.x, gridDim.x);
-  const int qt = lg % nqt, bh = lg / nqt;
+  int qt, bh;
+  query_tile(nqt, M, N, W, 16 * NW, qt, bh);
   const int b = bh / H, h = bh - b * H;
   const int kvh = h / (H / HKV);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
