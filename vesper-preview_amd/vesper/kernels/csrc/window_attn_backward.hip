@@ -421,8 +421,8 @@ void launch_backward(const T* q, const T* keys, const T* values, const T* o, con
   // waves a workgroup (16 queries a dQ wave, 16 KB keys a dK/dV wave); the dK/dV kernel's bound
   // asks for 2 waves a SIMD at least (256 VGPRs): its D 64 instance takes 126 and so runs 4 (two
   // workgroups a CU). Two key blocks a wave (each Q, dO fragment feeding two MFMAs) took 202
-  // VGPRs, halving that, and ran slower (dK/dV 67 -> 77 us at B4 T4096 H8 d64 w512); two query blocks
-  // a dQ wave (168 VGPRs, three waves a SIMD) too (a backward 103 -> 113 us there).
+  // VGPRs, halving that, and ran slower (dK/dV 67 -> 77 us at B4 T4096 H8 d64 w512); so did two query
+  // blocks a dQ wave with it, both in 4-wave workgroups (a backward 111.5 -> 115.8 us there).
   constexpr int kDqWaves = 8, kDkvWaves = 8, kDkvWavesPerSimd = 2, kDkvBlocks = 1;
   const int nqt = (N + 16 * kDqWaves - 1) / (16 * kDqWaves);
   const int nkt = (M + N + 16 * kDkvWaves * kDkvBlocks - 1) / (16 * kDkvWaves * kDkvBlocks);
