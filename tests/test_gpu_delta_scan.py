@@ -533,6 +533,28 @@ def test_fp32_gradients_at_the_edges_of_a_chunk(dk, n):
     _grad_check(delta_scan_fused_fp32, _fp32_inputs(3, n, 5, dk), TOL_FP32, active=act)
 
 
+# The initial state's gradient, a float32 sum over every token's products. Its mean error over four seeds
+# with the products' k order as mm16 has it, and with k in blocks of 16: 4.11e-7 / 4.29e-7 at width 16,
+# 3.49e-7 / 3.56e-7 at 32, 2.49e-7 / 2.54e-7 at 128 (the same bits in every run); the bounds lie halfway.
+@pytest.mark.parametrize(("dk", "n", "h", "bound"), [(16, 1000, 8, 4.20e-7), (32, 700, 6, 3.525e-7),
+                                                     (128, 300, 3, 2.515e-7)])
+def test_the_float32_state_gradient_keeps_its_error_against_float64(dk, n, h, bound):
+    from vesper.kernels.delta_scan import delta_scan_fused_fp32
+
+    errors = []
+    for seed in range(4):
+        q, k, v, beta, h0 = scan_inputs(4, n, h, dk, seed)
+        q = torch.nn.functional.normalize(q, dim=-1)
+        g = torch.Generator().manual_seed(seed + 50)
+        d_o, d_s = torch.randn(4, n, h, dk, generator=g), torch.randn(4, h, dk, dk, generator=g)
+        ref = [t.double().requires_grad_() for t in (q, k, v, beta, h0)]
+        (want,) = torch.autograd.grad(delta_scan_chunked(*ref, 64), ref[4:], (d_o.double(), d_s.double()))
+        ins = [t.to(GPU).requires_grad_() for t in (q, k, v, beta, h0)]
+        (got,) = torch.autograd.grad(delta_scan_fused_fp32(*ins), ins[4:], (d_o.to(GPU), d_s.to(GPU)))
+        errors.append(relative_error(got, want))
+    assert sum(errors) / len(errors) < bound, errors
+
+
 # the shape the reference quotes both fused scans at (kernels/delta_scan.py:22-24, "stage-1 size":
 # b 32, n 88, h 2, dk 16), forward and every gradient against the float64 oracle; the reference
 # reports about 2e-7 relative for its fp32 scan there
