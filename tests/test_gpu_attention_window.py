@@ -230,3 +230,19 @@ def test_a_break_anywhere_in_the_positions_is_refused_and_the_next_call_runs(m, 
         return
     o, after = attend(q, k, k, pos[:, m:].to(GPU), cache)
     assert torch.equal(o, want[0]) and torch.equal(after.pos, want[1].pos)
+
+
+def test_attend_under_a_gpu_default_device():
+    from vesper.attention import KVCache, attend
+    from vesper.contracts import ContractError
+
+    g = torch.Generator().manual_seed(4)
+    q, k, ck = (torch.randn(2, r, 2, 16, generator=g).to(GPU, BF16) for r in (9, 9, 5))
+    pos = torch.arange(14).expand(2, 14).to(GPU)
+    cache = KVCache(ck, ck, pos[:, :5], 8)
+    want = attend(q, k, k, pos[:, 5:], cache)
+    with torch.device(GPU):
+        got = attend(q, k, k, pos[:, 5:], cache)
+        with pytest.raises(ContractError, match="consecutive"):
+            attend(q, k, k, pos[:, 5:] + 1, cache)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1].k, want[1].k) and torch.equal(got[1].pos, want[1].pos)

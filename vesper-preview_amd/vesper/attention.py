@@ -262,7 +262,7 @@ class _PositionsCheck:
     def __init__(self, cache_pos: Tensor, pos: Tensor) -> None:
         b, n = pos.shape
         self.inputs = cache_pos.contiguous(), pos.contiguous()
-        self.word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self.word = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
         self.done = torch.cuda.Event()
         stream = torch.cuda.current_stream(pos.device)
         with _lib.on_device(pos.device):
