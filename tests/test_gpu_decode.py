@@ -178,6 +178,24 @@ def test_the_decode_shape_b64_d512_h8_w512_two_passes():
         assert bool(torch.isfinite(y).all())
 
 
+@pytest.mark.parametrize("default", [torch.bfloat16, torch.float64])
+def test_the_step_does_not_depend_on_the_default_dtype(default):
+    from vesper.decode import cold_states, decode_step
+
+    column = _column(4, passes=2)
+    x = _inputs(2, 1, 64, seed=9).to(GPU)
+    flat = cold_states(column, 2, GPU)
+    want = decode_step(column, 2, [x, _at(0, 2), *[t.clone() for t in flat]])
+    try:
+        torch.set_default_dtype(default)
+        got = decode_step(column, 2, [x, _at(0, 2), *flat])  # the caller's own float32 states
+        cold = decode_step(column, 2, [x, _at(0, 2), *cold_states(column, 2, GPU)])
+    finally:
+        torch.set_default_dtype(torch.float32)
+    for a, b, c in zip(got, cold, want):
+        assert a.dtype == c.dtype and torch.equal(a, c) and torch.equal(b, c)
+
+
 def test_refusals():
     from vesper.contracts import ContractError
     from vesper.decode import CapturedDecoder, cold_states, decode_step

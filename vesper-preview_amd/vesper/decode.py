@@ -44,8 +44,8 @@ def cold_states(column: LoopedColumn, b: int, device: torch.device) -> list[Tens
     h, hkv, dk, w = column.heads, column.kv_heads, column.head_dim, column.window
     flat: list[Tensor] = []
     for _ in range(column.passes):
-        flat += [torch.zeros(b, h, dk, dk, device=device),
-                 torch.zeros(b, column.key_history, h * dk, device=device),
+        flat += [torch.zeros(b, h, dk, dk, dtype=torch.float32, device=device),
+                 torch.zeros(b, column.key_history, h * dk, dtype=torch.float32, device=device),
                  torch.zeros(b, w, hkv, dk, dtype=BF16, device=device),
                  torch.zeros(b, w, hkv, dk, dtype=BF16, device=device),
                  torch.zeros(b, w, dtype=torch.long, device=device),
@@ -126,7 +126,7 @@ def decode_step(column: LoopedColumn, depth: int, values: Sequence[Tensor],
             a, _ = ring_attention(aq, ak, av.view(b, 1, hkv, dk), position, ring, inplace=True, check_positions=False,
                                   workspace=workspace)
             pending = a.reshape(b, hd)
-        x = torch.empty(b, 1, d, device=xs.device)
+        x = torch.empty(b, 1, d, dtype=torch.float32, device=xs.device)
         residual_rows_where(xs.view(b, 1, d), pending.view(b, 1, d), x, None)  # float32 (promoted in the add)
     return [x, *flat]
 
