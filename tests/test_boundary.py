@@ -225,3 +225,20 @@ def test_the_reference_scan_backend_equals_the_oracle_scan():
 
     o16, s32 = recurrent_scan("reference", *(t.to(torch.bfloat16) for t in (q, k, v, beta)), s0.float())
     assert o16.dtype == torch.bfloat16 and s32.dtype == torch.float32
+
+
+def test_a_width_given_as_a_kind_of_int_is_checked_as_one():
+    import enum
+
+    from vesper.contracts import ContractError, check_shape
+
+    class Width(enum.IntEnum):
+        HEAD = 3
+
+    dims = {}
+    check_shape("t", torch.zeros(2, 3), ("b", Width.HEAD), dims)
+    assert dims == {"b": 2}
+    with pytest.raises(ContractError, match="axis 1 must be .*got 5"):
+        check_shape("t", torch.zeros(2, 5), ("b", Width.HEAD), {})
+    with pytest.raises(ContractError, match="axis 0"):
+        check_shape("t", torch.zeros(2, 5), (True, 5), {})

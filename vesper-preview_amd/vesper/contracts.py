@@ -28,7 +28,7 @@ def check_shape(name: str, tensor: torch.Tensor, spec: DimSpec, dims: Dims, dtyp
         raise ContractError(f"{name}: expected rank {len(spec)} {spec}, got shape {tuple(shape)}")
     bind = dims.setdefault
     for want, got in zip(spec, shape):
-        if (want if want.__class__ is int else bind(want, got)) != got:
+        if (want if isinstance(want, int) else bind(want, got)) != got:
             _refuse_shape(name, tuple(shape), spec, dims)
     if dtype is not None and tensor.dtype != dtype:
         raise ContractError(f"{name}: dtype must be {dtype}, got {tensor.dtype}")
