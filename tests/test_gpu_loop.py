@@ -312,3 +312,28 @@ def test_the_pass_end_takes_strided_sources():
     assert all(torch.equal(p, q) for p, q in zip(*results))
     with pytest.raises(ContractError):
         end_pass(x1, a, x, active, exits, torch.zeros(b, n, dtype=torch.int32, device=GPU), [(src, strided(dst))], norm=True)
+
+
+def test_the_pass_end_refuses_rows_outside_its_contract():
+    from vesper.contracts import ContractError
+    from vesper.kernels.carry import end_pass
+
+    def call(d, b=2, n=3, shift=None):
+        def rows(dtype, name):
+            t = torch.zeros(b * n * d + 1, dtype=dtype, device=GPU)
+            return (t[1:] if shift == name else t[:-1]).view(b, n, d)
+
+        flags = torch.ones(b, n, dtype=torch.bool, device=GPU)
+        return end_pass(rows(torch.float32, "x1"), rows(torch.bfloat16, "a"), rows(torch.float32, "x"), flags, None,
+                        torch.zeros(b, n, dtype=torch.int32, device=GPU), [], norm=True)
+
+    for d in (4, 12, 2056):
+        for n in (3, 0):  # without tokens too
+            with pytest.raises(ContractError, match="multiple of 8"):
+                call(d, n=n)
+    for name in ("x1", "a", "x"):
+        with pytest.raises(ContractError, match=f"{name} must be 16-byte aligned"):
+            call(16, shift=name)
+    nxt, out = call(16, n=0)
+    assert nxt.shape == (2, 0) and out is not None and out.shape == (2, 0, 16)
+    assert not bool(call(16)[0].any())

@@ -171,13 +171,18 @@ def end_pass(x1: Tensor, a: Tensor, x: Tensor, active: Tensor, exits: Tensor | N
             raise ContractError(f"item {i}: src {tuple(src.shape)} {src.dtype}, dst {tuple(dst.shape)} {dst.dtype}")
     if not all(t.is_contiguous() for t in (x, n_iters, *(dst for _, dst in freeze))):
         raise ContractError("x, n_iters and every freeze target must be contiguous (they are written in place)")
+    b, n, d = x1.shape
+    if d % 8 or not 8 <= d <= 2048:
+        raise ContractError(f"x1: width {d} is not a multiple of 8 in 8..2048")
     x1, a, active = x1.contiguous(), a.contiguous(), active.contiguous()
     exits_c = None if exits is None else exits.contiguous()
     sources = [src.contiguous() for src, _ in freeze]
-    if x.data_ptr() == x1.data_ptr():
-        raise ContractError("x must not be x1")
-    b, n, d = x1.shape
+    for name, t in (("x1", x1), ("a", a), ("x", x)):
+        if t.data_ptr() % 16:
+            raise ContractError(f"{name} must be 16-byte aligned")
     rows, count = b * n, len(freeze)
+    if rows and x.data_ptr() == x1.data_ptr():
+        raise ContractError("x must not be x1")
     nxt = torch.empty_like(active)
     out = torch.empty(b, n, d, dtype=torch.bfloat16, device=device) if norm else None
     if rows == 0:
