@@ -289,10 +289,12 @@ def test_the_reference_benchmark_shape_b16_n1024_m512_h8_hkv2_d64():
 
 # either side of each line of the launches: dK/dV in 4-wave workgroups up to 768 8-wave ones (48 batch rows
 # of 8 KV heads, two and three 128-key tiles; 97 over one), its heads a multiple of 8 or not; the query
-# tiles heavy first (512 workgroups or more, a quarter of the tiles before the window is full) or in order
+# tiles heavy first (a quarter of the tiles before the window is full above 512 workgroups, half at 512) or
+# in order
 @pytest.mark.parametrize(("b", "n", "m", "w", "h", "hkv"), [
     (48, 200, 56, 64, 8, 8), (48, 200, 57, 64, 8, 8), (97, 1000, 24, 100, 1, 1), (3, 200, 40, 64, 6, 3),
-    (8, 1000, 0, 512, 8, 2), (8, 897, 300, 512, 8, 4), (8, 1000, 500, 512, 8, 2), (9, 1025, 0, 129, 7, 7)])
+    (8, 1000, 0, 512, 8, 2), (8, 897, 300, 512, 8, 4), (8, 1000, 500, 512, 8, 2), (9, 1025, 0, 129, 7, 7),
+    (16, 500, 3, 129, 8, 2), (16, 500, 3, 257, 8, 2), (16, 601, 101, 512, 8, 2)])
 def test_the_gradients_on_either_side_of_the_launch_rules(b, n, m, w, h, hkv):
     q, keys, values = _inputs(b, n, m, h, hkv, 64, seed=n + m)
     up = torch.randn(b, n, h, 64, generator=torch.Generator().manual_seed(n)).to(BF16)
@@ -416,3 +418,24 @@ def test_carried_refusals():
         window_attention(q, keys, values, 8, active=active, carried=(keys, carried[1]))
     with pytest.raises(ContractError, match="carried holds"):
         window_attention(q, keys, values, 8, active=active, carried=carried[:1])
+
+
+# the query tiles heavy first (more than 512 workgroups and a quarter of the tiles or more short, 512 and
+# half) and in order (512 and a quarter; heads not a multiple of 8), with the keys from two sources
+@pytest.mark.parametrize("dk", [16, 64, 128, 256])
+@pytest.mark.parametrize(("b", "n", "m", "w", "h", "hkv"), [
+    (16, 601, 101, 512, 8, 2), (13, 601, 33, 300, 8, 4), (16, 500, 3, 257, 8, 8), (16, 500, 3, 129, 8, 2),
+    (75, 500, 70, 400, 3, 1)])
+def test_two_key_sources_in_either_order_of_the_query_tiles(dk, b, n, m, w, h, hkv):
+    from vesper.kernels.window_attn import window_attention, window_attention_cached
+
+    q, keys, values, carried, active = _carry_case(b, n, m, h, hkv, dk, seed=n + m)
+    mk, mv = _merged_kv(keys, values, carried, active)
+    want = window_attention(q, mk, mv, w, active=active)
+    assert torch.equal(window_attention(q, keys, values, w, active=active, carried=carried), want)
+    plain = window_attention(q, keys, values, w)
+    split = (keys[:, :m].contiguous(), values[:, :m].contiguous(), keys[:, m:].contiguous(), values[:, m:].contiguous())
+    assert torch.equal(window_attention_cached(q, *split, w), plain)
+    for rows in (slice(0, 1), slice(b - 1, b)):
+        cpu = [t[rows].float().cpu() for t in (q, keys, values)]
+        assert relative_error(plain[rows], oracle_window(*cpu, w)) < 1e-2

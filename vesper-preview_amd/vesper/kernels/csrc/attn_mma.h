@@ -3,6 +3,8 @@
 #pragma once
 #include "common.h"
 
+#include <algorithm>
+
 namespace vsp {
 namespace {
 
@@ -39,26 +41,35 @@ __device__ __forceinline__ float max_over_groups(float x) {
   return fmax_ieee(__uint_as_float(c[0]), __uint_as_float(c[1]));
 }
 
-// The workgroup's query tile (of nqt of QT queries) and (batch, head) of a kernel that walks each
-// query's window of W keys. A head's tiles run on one XCD, in order: their key windows overlap, so most
-// of each tile's K and V reads hit that XCD's L2. The first tiles see fewer than W keys. Where they are
-// a quarter of a head's tiles or more and a CU holds two workgroups or more, in that order some CUs get
-// several heavy tiles and others light ones; there the heavy tiles go first, the XCD's heads taking
-// turns (plain attention, in order / heavy first, us: B16 N1024 H8 30.2 / 27.1, B8 N1024 H8 over 2 20.2 /
-// 18.7, B9 N1024 M300 H8 24.8 / 21.8, B8 N2048 H8 31.4 / 30.4). Longer sequences keep the order, whose
-// K and V reuse counts for more there (B4 N4096 H8 31.5 / 33.2).
-__device__ __forceinline__ void query_tile(int nqt, int M, int N, int W, int QT, int& qt, int& bh) {
-  const int heads = (int)gridDim.x / nqt;
-  const int light = (max(min(W, M + N) - 1 - M, 0) + QT - 1) / QT;
-  if (heads % 8 == 0 && gridDim.x >= 512 && 4 * light >= nqt) {
-    const int per = heads >> 3, r = (int)blockIdx.x >> 3, rank = r / per;
-    bh = (int)(blockIdx.x & 7) * per + (r - rank * per);
-    qt = nqt - 1 - rank;
-  } else {
-    const int lg = xcd_logical_block(blockIdx.x, gridDim.x);
-    bh = lg / nqt;
-    qt = lg - bh * nqt;
-  }
+constexpr size_t kCus = 256;  // of an MI355X
+
+// The order of the query tiles (nqt a head, QT queries each) of a kernel that walks each query's window of
+// W keys, as query_tile takes it; decided on the host, so that a workgroup divides once before its first
+// load (deciding in the kernel cost the in-order shapes about 1 %).
+// In order (0): a head's tiles run on one XCD one after the other. Their key windows overlap, so most of
+// each tile's K and V reads hit that XCD's L2.
+// Heavy first (the heads of an XCD): the first tiles see fewer than W keys. Where they are a quarter of a
+// head's tiles or more, in order some CUs get several full tiles and others short ones; the full ones
+// first, the XCD's heads taking turns, even that out once a CU has more than two workgroups. With exactly
+// two, full tiles still meet unless half of them are short. Longer sequences keep the order, whose K and V
+// reuse counts for more there. In order / heavy first at D 64, us: plain B16 N1024 H8 31.2 / 27.9, B8 N1024
+// H8 over 2 20.8 / 18.8, B9 N1024 M300 H8 26.3 / 23.4, B8 N2048 H8 32.0 / 31.4; cached B9 N1024 M300 26.0 /
+// 23.6; carried B16 N1024 H8 45.9 / 35.2; forward and backward B16 N1024 H8 134.7 / 124.7. Other widths, B16
+// N1024 H8, plain: 16 23.8 / 19.3, 32 23.4 / 20.3, 128 55.7 / 51.3, 256 167.7 / 144.8. Two a CU and a quarter
+// short (B4 N2048 H8): 16 carried 17.0 / 17.4, 256 plain 87.9 / 89.9; 64 the same.
+inline int query_order(size_t heads, int nqt, int M, int N, int W, int QT) {
+  const int64_t light = (std::max<int64_t>(std::min<int64_t>(W, (int64_t)M + N) - 1 - M, 0) + QT - 1) / QT;
+  const size_t workgroups = heads * nqt;
+  const bool uneven = workgroups > 2 * kCus ? 4 * light >= nqt : workgroups == 2 * kCus && 2 * light >= nqt;
+  return uneven && heads % 8 == 0 ? (int)(heads / 8) : 0;
+}
+// The workgroup's query tile and (batch, head) in that order: one division for both orders.
+__device__ __forceinline__ void query_tile(int nqt, int order, int& qt, int& bh) {
+  const bool heavy = order != 0;  // the XCD's heads take turns, each from its last tile on
+  const unsigned x = heavy ? blockIdx.x >> 3 : (unsigned)xcd_logical_block(blockIdx.x, gridDim.x);
+  const unsigned per = (unsigned)(heavy ? order : nqt), quotient = x / per, rest = x - quotient * per;
+  qt = heavy ? nqt - 1 - (int)quotient : (int)rest;
+  bh = heavy ? (int)((blockIdx.x & 7) * per + rest) : (int)quotient;
 }
 
 }  // namespace

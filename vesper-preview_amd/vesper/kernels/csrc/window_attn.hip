@@ -49,7 +49,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPla
                                                              float* __restrict__ lse,
                                                              const uint8_t* __restrict__ active, const T* keys_c,
                                                              const T* values_c, int N, int M, int H,
-                                                             int HKV, int W, float scale_log2, int nqt) {
+                                                             int HKV, int W, float scale_log2, int nqt, int order) {
   using V8 = typename Mma<T>::V8;
   using V4 = typename Mma<T>::V4;
   constexpr bool CARRY = SRC == kSrcCarried, CACHED = SRC == kSrcCached;
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPla
 
   auto kswz = [](int row) { return kSwzK ? 2 * ((row >> 1) & 3) : 0; };  // K's segment swizzle
   int qt, bh;
-  query_tile(nqt, M, N, W, QT, qt, bh);
+  query_tile(nqt, order, qt, bh);
   const int b = bh / H, h = bh - b * H;
   const int kvh = h / (H / HKV);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -431,12 +431,13 @@ template <typename T, int SRC>
 void launch_window(dim3 grid, hipStream_t stream, const T* q, const T* keys, const T* values, T* o, float* lse,
                    const uint8_t* active, const T* kc, const T* vc, int N, int M, int H, int HKV, int D, int W,
                    float scale_log2, int nqt) {
+  const int order = query_order(grid.x / nqt, nqt, M, N, W, 128);
   switch (D) {
-    case 16: hipLaunchKernelGGL((window_attn_kernel<T, 16, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt); break;
-    case 32: hipLaunchKernelGGL((window_attn_kernel<T, 32, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt); break;
-    case 64: hipLaunchKernelGGL((window_attn_kernel<T, 64, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt); break;
-    case 128: hipLaunchKernelGGL((window_attn_kernel<T, 128, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt); break;
-    default: hipLaunchKernelGGL((window_attn_kernel<T, 256, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt); break;
+    case 16: hipLaunchKernelGGL((window_attn_kernel<T, 16, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order); break;
+    case 32: hipLaunchKernelGGL((window_attn_kernel<T, 32, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order); break;
+    case 64: hipLaunchKernelGGL((window_attn_kernel<T, 64, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order); break;
+    case 128: hipLaunchKernelGGL((window_attn_kernel<T, 128, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order); break;
+    default: hipLaunchKernelGGL((window_attn_kernel<T, 256, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order); break;
   }
 }
 

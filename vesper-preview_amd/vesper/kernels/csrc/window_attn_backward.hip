@@ -96,7 +96,7 @@ __global__ __launch_bounds__(64 * NW) void attn_dq_kernel(const T* __restrict__ 
                                                       const T* __restrict__ values, const T* __restrict__ o,
                                                       const T* __restrict__ dout, const float* __restrict__ lse,
                                                       float* __restrict__ dsum, T* __restrict__ dq, int N, int M,
-                                                      int H, int HKV, int W, float scale, float scale_log2, int nqt) {
+                                                      int H, int HKV, int W, float scale, float scale_log2, int nqt, int order) {
   using Sh = BwdShape<D>;
   using V8 = typename Mma<T>::V8;
   using V4 = typename Mma<T>::V4;
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(64 * NW) void attn_dq_kernel(const T* __restrict__ 
   __shared__ __align__(16) T sK[2][KT * Sh::P];
   __shared__ __align__(16) T sV[2][KT * Sh::P];
   int qt, bh;
-  query_tile(nqt, M, N, W, 16 * NW, qt, bh);
+  query_tile(nqt, order, qt, bh);
   const int b = bh / H, h = bh - b * H;
   const int kvh = h / (H / HKV);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -428,7 +428,8 @@ void launch_backward(const T* q, const T* keys, const T* values, const T* o, con
   const int nkt = (M + N + 16 * kDkvWaves * kDkvBlocks - 1) / (16 * kDkvWaves * kDkvBlocks);
   hipLaunchKernelGGL((attn_dq_kernel<T, D, kDqWaves>), dim3((unsigned)((size_t)nqt * H * B)), dim3(64 * kDqWaves), 0,
                      stream, q, keys,
-                     values, o, dout, lse, dsum, dq, N, M, H, HKV, W, scale, scale_log2, nqt);
+                     values, o, dout, lse, dsum, dq, N, M, H, HKV, W, scale, scale_log2, nqt,
+                     query_order((size_t)H * B, nqt, M, N, W, 16 * kDqWaves));
   auto dkv = [&](auto waves, int tiles) {
     hipLaunchKernelGGL((attn_dkv_kernel<T, D, decltype(waves)::value, kDkvWavesPerSimd, kDkvBlocks>),
                        dim3((unsigned)((size_t)tiles * HKV * B)), dim3(64 * decltype(waves)::value), 0, stream, q, keys,
