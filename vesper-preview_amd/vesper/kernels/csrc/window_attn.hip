@@ -189,7 +189,20 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPla
           continue;
         }
       }
-      if constexpr (kDirect && (CARRY || CACHED)) {
+      if constexpr (CARRY && D >= 256) {
+        // one workgroup a CU: a lane's own 64-bit source address costs no registers that another workgroup
+        // would use, and two turns of loads cost more (B8 N2048 H8 205.9 us against 211.8); rows past the
+        // last key re-read key S - 1, from that key's own source
+        const int ins = w + 4 * j;
+        const int pos = ins * 64 + l;
+        const int row = pos / PSEG, seg = pos - row * PSEG;
+        const int rowv = pos / PSEGV, segv = pos - rowv * PSEGV;
+        const int key = min(k0 + row, S - 1), keyv = min(k0 + rowv, S - 1);
+        const size_t sk = (size_t)key * kv_row + 8 * (seg < SEG ? seg ^ kswz(row) : 0);
+        const size_t sv = (size_t)keyv * kv_row + 8 * (segv < SEG ? segv : 0);
+        if (ins < NINS) load_lds16((((fresh >> (key - k0)) & 1) ? kbase : kcbase) + sk, Kn + ins * 64 * 8);
+        if (ins < NINSV) load_lds16((((fresh >> (keyv - k0)) & 1) ? vbase : vcbase) + sv, Vn + ins * 64 * 8);
+      } else if constexpr (kDirect && (CARRY || CACHED)) {
         // Per-lane sources: a buffer resource is one for the wave, so the lanes of each source load
         // in turn under the execution mask (a direct load writes a lane's 16 bytes to the lane's own
         // place, whichever lanes take part). Rows past the last key read zeros, as plainly loaded
