@@ -288,16 +288,20 @@ def test_the_reference_benchmark_shape_b16_n1024_m512_h8_hkv2_d64():
 
 
 # either side of each line of the launches: dK/dV in 4-wave workgroups up to 768 8-wave ones (48 batch rows
-# of 8 KV heads, two and three 128-key tiles; 97 over one), its heads a multiple of 8 or not; the query
-# tiles heavy first (a quarter of the tiles before the window is full above 512 workgroups, half at 512) or
-# in order
+# of 8 KV heads, two and three 128-key tiles; 97 over one), and at width 64 between 384 and 576 only where
+# many keys are short of queries and the heads are a multiple of 8 (48 rows of eight tiles, 56 with a short
+# and a long window, 57 and 72); the query tiles heavy first (a quarter of the tiles before the window is
+# full above 512 workgroups, half at 512) or in order
+@pytest.mark.parametrize("dk", [64, 16])
 @pytest.mark.parametrize(("b", "n", "m", "w", "h", "hkv"), [
     (48, 200, 56, 64, 8, 8), (48, 200, 57, 64, 8, 8), (97, 1000, 24, 100, 1, 1), (3, 200, 40, 64, 6, 3),
+    (48, 1000, 0, 64, 1, 1), (56, 1000, 0, 64, 1, 1), (56, 990, 34, 512, 1, 1), (57, 1000, 0, 512, 1, 1),
+    (72, 1000, 0, 64, 1, 1),
     (8, 1000, 0, 512, 8, 2), (8, 897, 300, 512, 8, 4), (8, 1000, 500, 512, 8, 2), (9, 1025, 0, 129, 7, 7),
     (16, 500, 3, 129, 8, 2), (16, 500, 3, 257, 8, 2), (16, 601, 101, 512, 8, 2)])
-def test_the_gradients_on_either_side_of_the_launch_rules(b, n, m, w, h, hkv):
-    q, keys, values = _inputs(b, n, m, h, hkv, 64, seed=n + m)
-    up = torch.randn(b, n, h, 64, generator=torch.Generator().manual_seed(n)).to(BF16)
+def test_the_gradients_on_either_side_of_the_launch_rules(b, n, m, w, h, hkv, dk):
+    q, keys, values = _inputs(b, n, m, h, hkv, dk, seed=n + m)
+    up = torch.randn(b, n, h, dk, generator=torch.Generator().manual_seed(n)).to(BF16)
     got = _grads(q, keys, values, w, up)
     want = _oracle_grads(q, keys, values, w, up, dtype=torch.float32)
     for a, x, name in zip(got, want, ("o", "dq", "dk", "dv")):

@@ -20,7 +20,7 @@
 // Both launch 8 waves a workgroup: a staged tile then serves 128 queries (keys), against 64 at 4
 // waves, which cuts the window's overlap re-fetch about in half (dq 69.7 -> 62.0 us, dkv 97.2 ->
 // 86.5 us at B4 T4096 H8 d64 w512); 16 waves measured slower for both. Where that leaves the dK/dV
-// kernel with few workgroups, it runs 4 waves (launch_backward).
+// kernel with few workgroups, it runs 4 waves (dkv_in_fours).
 #include "attn_mma.h"
 #include "common.h"
 #include "vesper_kernels.h"
@@ -414,6 +414,26 @@ __global__ __launch_bounds__(64 * NW, WAVES_PER_SIMD) void attn_dkv_kernel(const
   }
 }
 
+// Whether dK/dV runs in 4-wave workgroups (nkt 8-wave tiles a KV head). Up to three 8-wave workgroups a
+// CU, a workgroup's chain of steps (the group's heads times its query tiles, one after the other) and the
+// CUs' unequal shares set the time: half the keys a workgroup make the chain shorter and the shares more
+// even. Beyond, the tiles' staging counts for more. A whole backward with its forward, 8 / 4 waves, us, at D
+// 64: B16 N1024 M512 H8 over 2 (384 workgroups) 159.9 / 135.8, B3 N4096 H6 (576) 108.6 / 102.0, B8 N1024
+// M512 H8 (768) 91.3 / 81.2; at 16 61.2 / 50.3 for the last. At D 64 between 1.5 and 2.25 workgroups a CU, 8
+// waves run all of them at once with even shares, and the staging decides: B2 N4096 H8 (512) 74.9 / 80.1,
+// B7 N2048 H4 (448) 73.9 / 79.3, B1 N8000 M512 H8 (536) 75.6 / 81.0; unless two fifths of the keys or more
+// are seen by fewer than W queries (those of the cache and the last window) and the heads fill the XCDs
+// evenly: B8 N1024 H8 (512) 70.2 / 69.0, B8 N512 M512 H8 (512) 57.3 / 52.7, 40 heads of N1024 M512 (480) 72.7
+// / 67.9 (but 42 heads 72.9 / 77.7). At D 16 and 32 the tiles are cheap to stage: there 51.8 / 50.2 and 54.4
+// / 52.8 at B4 N2048 H8 (512). Wider heads fill the LDS with two workgroups of either size.
+template <int D>
+bool dkv_in_fours(int B, int N, int M, int HKV, int W, int nkt) {
+  const size_t heads = (size_t)B * HKV, workgroups = heads * nkt;
+  if (D == 64 && workgroups > 3 * kCus / 2 && workgroups < 9 * kCus / 4)
+    return heads % 8 == 0 && 5 * ((int64_t)M + std::min(W, N)) >= 2 * ((int64_t)M + N);
+  return workgroups <= 3 * kCus;
+}
+
 template <typename T, int D>
 void launch_backward(const T* q, const T* keys, const T* values, const T* o, const T* dout, const float* lse, float* dsum,
                      T* dq, T* dk, T* dv, int B, int N, int M, int H, int HKV, int W, float scale, hipStream_t stream) {
@@ -435,17 +455,10 @@ void launch_backward(const T* q, const T* keys, const T* values, const T* o, con
                        dim3((unsigned)((size_t)tiles * HKV * B)), dim3(64 * decltype(waves)::value), 0, stream, q, keys,
                        values, dout, lse, dsum, dk, dv, N, M, H, HKV, W, scale, scale_log2, tiles);
   };
-  // Up to three 8-wave workgroups a CU, a workgroup's chain of steps (the group's heads times its query
-  // tiles, one after the other) and the CUs' unequal shares set the time: half the keys a workgroup make
-  // the chain shorter and the shares more even. Beyond, the tiles' staging counts for more. A whole
-  // backward, 8 / 4 waves, us: B16 N1024 M512 H8 over 2 (384 workgroups) 128.9 / 106.1, B8 N1024 H8 over
-  // 2 (128) 86.4 / 75.8, B3 N4096 H6 (576) 83.7 / 76.4, B8 N1024 M512 H8 (768) 69.8 / 59.1, B4 N4096 H8
-  // (1024) 103.1 / 105.7, B8 N2048 H8 (1024) 102.0 / 104.9. Wider heads fill the LDS with two workgroups
-  // of either size.
-  if (D <= 64 && (size_t)nkt * HKV * B <= 768)
-    dkv(std::integral_constant<int, kDkvWaves / 2>{}, (M + N + 16 * kDkvWaves / 2 - 1) / (16 * kDkvWaves / 2));
-  else
-    dkv(std::integral_constant<int, kDkvWaves>{}, nkt);
+  if constexpr (D <= 64)
+    if (dkv_in_fours<D>(B, N, M, HKV, W, nkt))
+      return dkv(std::integral_constant<int, kDkvWaves / 2>{}, (M + N + 16 * kDkvWaves / 2 - 1) / (16 * kDkvWaves / 2));
+  dkv(std::integral_constant<int, kDkvWaves>{}, nkt);
 }
 
 template <typename T>
