@@ -263,9 +263,11 @@ def test_the_form_picked_by_shape_matches_the_oracle(b, n, h):
 
 
 # 17 and 18 segments (an odd and an even number of folded maps), 31; either side of the line below
-# which the chains run (39 and 40 chunks of one head), each also one token off a whole chunk
+# which the chains run (39 and 40 chunks of one head, 52 and 56 of 32), each also one token off a
+# whole chunk
 @pytest.mark.parametrize(("b", "n", "h"), [(1, 68 * 64 - 1, 1), (1, 72 * 64, 1), (1, 124 * 64 - 63, 1),
-                                           (1, 38 * 64 + 1, 1), (1, 39 * 64 + 1, 1), (5, 4033, 8)])
+                                           (1, 38 * 64 + 1, 1), (1, 39 * 64 + 1, 1), (5, 4033, 8),
+                                           (4, 52 * 64, 8), (4, 55 * 64 + 1, 8)])
 def test_long_sequences_of_few_heads_by_shape_match_the_oracle_and_the_chains(b, n, h):
     from vesper.kernels.delta_scan import delta_scan_fused
 

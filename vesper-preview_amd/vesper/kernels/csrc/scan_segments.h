@@ -71,14 +71,17 @@ constexpr size_t kSegMapBytes = 2 * 64 * 64 * sizeof(float);  // X and M of one 
 // Whether the segments outrun the value-slice chains. Past one chain workgroup a CU (four a head)
 // the chains queue, and the segments win. Below that, in tenths of a microsecond: a chain takes about
 // 6 a chunk; the two passes take about 110 more to start than it, 22 a chunk of a segment (8 the
-// maps, 14 the outputs) and 3 a map folded. Measured chains / segments, us: B H 12, T 2048 28.2 /
-// 30.2, T 4096 47.0 / 39.0, T 8191 83.3 / 50.4; B H 40, T 4096 54.5 / 52.0; B H 48, T 4096 55.2 /
-// 56.8, T 8191 92.9 / 88.2; B H 64, T 4096 60.1 / 65.6.
+// maps, 14 the outputs) and 3 a map folded; and 24 more from 25 to 36 heads, where seven to ten segments a
+// head nearly fill the CUs in either pass. Measured chains / segments, us, B H heads: 1 T 2560 30.6 / 26.2;
+// 12 T 4096 47.3 / 38.8, T 8191 83.4 / 49.4; 24 T 2560 36.9 / 36.0; 28 T 3072 41.1 / 42.6, T 3328 43.7 / 42.9;
+// 32 T 3072 41.7 / 44.4, T 3584 46.4 / 45.7, T 4096 51.0 / 47.5; 40 T 4096 58.1 / 52.7; 48 T 4096 56.9 / 56.0,
+// T 8191 102.4 / 89.8; 64 T 4096 59.0 / 65.2. Recording the states or reading carried rows moves neither line.
 inline bool seg_faster(int B, int H, int T) {
-  if ((long)B * H * 4 > kSegBlocks) return true;
+  const long heads = (long)B * H;
+  if (heads * 4 > kSegBlocks) return true;
   const SegShape sh = seg_shape(B, H, T);
   const int nc = (T + kChunk - 1) / kChunk;
-  return 6L * nc > 110 + 22L * sh.seglen + 3L * sh.nseg;
+  return 6L * nc > 110 + 22L * sh.seglen + 3L * sh.nseg + (heads > 24 && heads <= 36 ? 24 : 0);
 }
 
 template <int MODE, bool CARRY>
