@@ -1092,7 +1092,7 @@ def main() -> int:
                         "+ delta scan + window attention (w512) with bf16 projections (fixed N(0, 1/512) weights), "
                         "p_halt 0.3, copy-forward of halted tokens",
             "tok_s": round(looped["tok_s"], 1), "ms": round(looped["ms"], 3),
-            "copy_forward": "fused into the kernels' loads; one row-copy launch per pass",
+            "copy_forward": "fused into the kernels' loads; one launch ends a pass",
             "ms_with_where_merges": round(looped["ms_where"], 3),
             "ms_captured": round(looped["ms_captured"], 3),
             "mean_active_passes": round(looped["mean_passes"], 3),

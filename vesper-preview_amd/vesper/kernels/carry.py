@@ -1,11 +1,15 @@
-"""The looped column's copy-forward bookkeeping on MI355X: flagged token rows copied in place.
+"""The looped column's copy-forward bookkeeping on MI355X.
+
+``end_pass`` is what the column's pass loop runs (``vsp_pass_end``): the halting bookkeeping, the
+tokens halting now freezing their projections into the carried ones (``vesper/loop.py:523-537``,
+``_merge``), the hidden state of the tokens still in the loop (``vesper/loop.py:441-452``) and the next
+pass's norm, in one launch. ``halt_step`` and ``residual_rows_where`` are two of its parts as launches of
+their own, for the loop with ``where`` merges and the decoder's last add.
 
 ``copy_rows_where(items)`` performs, for each ``(src, dst, flags)``, ``dst[flags] = src[flags]``
 over the leading ``[b, n]`` token dimensions, every item in one kernel launch
-(``vsp_copy_rows_where``). It stands in for the row-wise ``where`` selects of the reference's
-pass loop: the freezing of the projections of the tokens that halt now into the carried ones
-(``vesper/loop.py:523-537``, ``_merge``) and the carried hidden state of halted tokens
-(``vesper/loop.py:441-452``). Only flagged rows are read and written.
+(``vsp_copy_rows_where``): the freezing alone, for a caller with a pass loop of its own (the package's
+loop does not call it). Only flagged rows are read and written.
 """
 
 from __future__ import annotations

@@ -59,9 +59,8 @@ __device__ __forceinline__ int tile_col() { return threadIdx.x & 15; }
 // put() converts and writes them to LDS. A kernel fetches every operand before it puts the first,
 // so all its loads are in flight together: with one workgroup per CU nothing else hides a load's
 // latency. Loads are unconditional (rows past N re-read row N - 1, selected to zero in put()), so
-// none sits behind a per-lane branch, which would make it wait for every earlier load. The kernels
-// run 256 threads a workgroup.
-constexpr int kThreads = 256;
+// none sits behind a per-lane branch, which would make it wait for every earlier load. NTH: the
+// workgroup's threads.
 
 template <typename TIn>
 __device__ __forceinline__ void load4_f32(const TIn* p, float (&x)[4]) {
@@ -79,7 +78,7 @@ __device__ __forceinline__ void load4_f32(const TIn* p, float (&x)[4]) {
 
 // chunk rows t0 .. t0 + 63 of a [B, N, H, D] tensor (head h of batch row b) into LDS [64][ld] as
 // fp32; rows past N are zero, and with `active` so are inactive tokens' rows
-template <typename TIn, int D, int NTH = kThreads>
+template <typename TIn, int D, int NTH>
 struct ChunkRows {
   typedef TIn V4 __attribute__((ext_vector_type(4)));
   static constexpr int kN = kC * D / 4, kIt = (kN + NTH - 1) / NTH;
@@ -125,7 +124,7 @@ struct ChunkBeta {
 };
 
 // a [R][D] fp32 global matrix (row pitch D) into LDS [R][ld]
-template <int R, int D, int NTH = kThreads>
+template <int R, int D, int NTH>
 struct MatRows {
   static constexpr int kN = R * D / 4, kIt = (kN + NTH - 1) / NTH;
   f32x4 raw[kIt];
@@ -145,7 +144,7 @@ struct MatRows {
 
 // a [D][D] fp32 matrix stored in accumulator order (accfrag: value slice s = column tile) into
 // LDS [D][ld], row-major
-template <int D, int NTH = kThreads>
+template <int D, int NTH>
 struct AccRows {
   static constexpr int NT = D / 16, kN = D * D / 4, kIt = (kN + NTH - 1) / NTH;
   f32x4 raw[kIt];
@@ -653,7 +652,7 @@ __global__ __launch_bounds__(kChunkThreads<D>) void scan_bwd_chunk_kernel(
     for (int r = 0; r < 4; ++r) Bd[(r0 + tile_row(r)) * PD + 16 * ct + tile_col()] = acc[r];
   }
   __syncthreads();
-  // dK accumulates in registers: the wave's rows r0, its column tiles ch, ch + 2
+  // dK accumulates in registers: the wave's rows r0, its column tiles ch, ch + NCH, ...
   f32x4 dka[NTW];
   // dDelta = K G + P^T dO (registers), dK = Delta G^T
   f32x4 ddl[NTW];
