@@ -44,8 +44,10 @@ __device__ __forceinline__ float max_over_groups(float x) {
 constexpr size_t kCus = 256;  // of an MI355X
 
 // The order of the query tiles (nqt a head, QT queries each) of a kernel that walks each query's window of
-// W keys, as query_tile takes it; decided on the host, so that a workgroup divides once before its first
-// load (deciding in the kernel cost the in-order shapes about 1 %).
+// W keys, as query_tile takes it; decided on the host and a template parameter of the kernels, so that
+// the in-order kernels are what they would be without the other order (with the choice in the kernel, even
+// of one precomputed value, they ran up to 1.5 % longer: 8 workgroups 4.90 -> 4.96 us, B4 N4096 H8 d256 178.8
+// -> 181.7).
 // In order (0): a head's tiles run on one XCD one after the other. Their key windows overlap, so most of
 // each tile's K and V reads hit that XCD's L2.
 // Heavy first (the heads of an XCD): the first tiles see fewer than W keys. Where they are a quarter of a
@@ -63,13 +65,18 @@ inline int query_order(size_t heads, int nqt, int M, int N, int W, int QT) {
   const bool uneven = workgroups > 2 * kCus ? 4 * light >= nqt : workgroups == 2 * kCus && 2 * light >= nqt;
   return uneven && heads % 8 == 0 ? (int)(heads / 8) : 0;
 }
-// The workgroup's query tile and (batch, head) in that order: one division for both orders.
+// The workgroup's query tile and (batch, head) in that order (HEAVY: it is not 0).
+template <bool HEAVY>
 __device__ __forceinline__ void query_tile(int nqt, int order, int& qt, int& bh) {
-  const bool heavy = order != 0;  // the XCD's heads take turns, each from its last tile on
-  const unsigned x = heavy ? blockIdx.x >> 3 : (unsigned)xcd_logical_block(blockIdx.x, gridDim.x);
-  const unsigned per = (unsigned)(heavy ? order : nqt), quotient = x / per, rest = x - quotient * per;
-  qt = heavy ? nqt - 1 - (int)quotient : (int)rest;
-  bh = heavy ? (int)((blockIdx.x & 7) * per + rest) : (int)quotient;
+  if constexpr (HEAVY) {  // the XCD's heads take turns, each from its last tile on
+    const int r = (int)blockIdx.x >> 3, rank = r / order;
+    bh = (int)(blockIdx.x & 7) * order + (r - rank * order);
+    qt = nqt - 1 - rank;
+  } else {
+    const int lg = xcd_logical_block(blockIdx.x, gridDim.x);
+    qt = lg % nqt;
+    bh = lg / nqt;
+  }
 }
 
 }  // namespace

@@ -24,6 +24,8 @@
 #include "common.h"
 #include "vesper_kernels.h"
 
+#include <type_traits>
+
 namespace vsp {
 namespace {
 
@@ -43,7 +45,7 @@ constexpr float kLazy = 8.f;
 // against 22.7 / 71.6, plain 21.6 / 65.5). Three workgroups per CU at D 64 instead of four: within 128
 // registers both variants spill 49 (29 and 45 us at 336).
 constexpr int kSrcPlain = 0, kSrcCarried = 1, kSrcCached = 2;
-template <typename T, int D, int SRC>
+template <typename T, int D, int SRC, bool HEAVY>
 __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPlain && D == 64 ? 3 : 4))) void window_attn_kernel(const T* __restrict__ q, const T* __restrict__ keys,
                                                              const T* __restrict__ values, T* __restrict__ o,
                                                              float* __restrict__ lse,
@@ -83,7 +85,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPla
 
   auto kswz = [](int row) { return kSwzK ? 2 * ((row >> 1) & 3) : 0; };  // K's segment swizzle
   int qt, bh;
-  query_tile(nqt, order, qt, bh);
+  query_tile<HEAVY>(nqt, order, qt, bh);
   const int b = bh / H, h = bh - b * H;
   const int kvh = h / (H / HKV);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -440,18 +442,30 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : (D >= 128 ? 2 : (SRC != kSrcPla
 
 bool attn_width(int D) { return D == 16 || D == 32 || D == 64 || D == 128 || D == 256; }
 
+template <typename T, int SRC, bool HEAVY>
+void launch_order(dim3 grid, hipStream_t stream, const T* q, const T* keys, const T* values, T* o, float* lse,
+                  const uint8_t* active, const T* kc, const T* vc, int N, int M, int H, int HKV, int D, int W,
+                  float scale_log2, int nqt, int order) {
+  auto launch = [&](auto width) {
+    hipLaunchKernelGGL((window_attn_kernel<T, decltype(width)::value, SRC, HEAVY>), grid, dim3(256), 0, stream, q, keys,
+                       values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order);
+  };
+  switch (D) {
+    case 16: launch(std::integral_constant<int, 16>{}); break;
+    case 32: launch(std::integral_constant<int, 32>{}); break;
+    case 64: launch(std::integral_constant<int, 64>{}); break;
+    case 128: launch(std::integral_constant<int, 128>{}); break;
+    default: launch(std::integral_constant<int, 256>{}); break;
+  }
+}
+
 template <typename T, int SRC>
 void launch_window(dim3 grid, hipStream_t stream, const T* q, const T* keys, const T* values, T* o, float* lse,
                    const uint8_t* active, const T* kc, const T* vc, int N, int M, int H, int HKV, int D, int W,
                    float scale_log2, int nqt) {
   const int order = query_order(grid.x / nqt, nqt, M, N, W, 128);
-  switch (D) {
-    case 16: hipLaunchKernelGGL((window_attn_kernel<T, 16, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order); break;
-    case 32: hipLaunchKernelGGL((window_attn_kernel<T, 32, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order); break;
-    case 64: hipLaunchKernelGGL((window_attn_kernel<T, 64, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order); break;
-    case 128: hipLaunchKernelGGL((window_attn_kernel<T, 128, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order); break;
-    default: hipLaunchKernelGGL((window_attn_kernel<T, 256, SRC>), grid, dim3(256), 0, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, W, scale_log2, nqt, order); break;
-  }
+  auto* launch = order != 0 ? launch_order<T, SRC, true> : launch_order<T, SRC, false>;
+  launch(grid, stream, q, keys, values, o, lse, active, kc, vc, N, M, H, HKV, D, W, scale_log2, nqt, order);
 }
 
 template <typename T>

@@ -91,7 +91,7 @@ __device__ __forceinline__ typename Mma<T>::V8 tr_frag(const T* tile, int r0, in
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-template <typename T, int D, int NW>
+template <typename T, int D, int NW, bool HEAVY>
 __global__ __launch_bounds__(64 * NW) void attn_dq_kernel(const T* __restrict__ q, const T* __restrict__ keys,
                                                       const T* __restrict__ values, const T* __restrict__ o,
                                                       const T* __restrict__ dout, const float* __restrict__ lse,
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(64 * NW) void attn_dq_kernel(const T* __restrict__ 
   __shared__ __align__(16) T sK[2][KT * Sh::P];
   __shared__ __align__(16) T sV[2][KT * Sh::P];
   int qt, bh;
-  query_tile(nqt, order, qt, bh);
+  query_tile<HEAVY>(nqt, order, qt, bh);
   const int b = bh / H, h = bh - b * H;
   const int kvh = h / (H / HKV);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -446,10 +446,14 @@ void launch_backward(const T* q, const T* keys, const T* values, const T* o, con
   constexpr int kDqWaves = 8, kDkvWaves = 8, kDkvWavesPerSimd = 2, kDkvBlocks = 1;
   const int nqt = (N + 16 * kDqWaves - 1) / (16 * kDqWaves);
   const int nkt = (M + N + 16 * kDkvWaves * kDkvBlocks - 1) / (16 * kDkvWaves * kDkvBlocks);
-  hipLaunchKernelGGL((attn_dq_kernel<T, D, kDqWaves>), dim3((unsigned)((size_t)nqt * H * B)), dim3(64 * kDqWaves), 0,
-                     stream, q, keys,
-                     values, o, dout, lse, dsum, dq, N, M, H, HKV, W, scale, scale_log2, nqt,
-                     query_order((size_t)H * B, nqt, M, N, W, 16 * kDqWaves));
+  const int order = query_order((size_t)H * B, nqt, M, N, W, 16 * kDqWaves);
+  auto dq_in = [&](auto heavy) {
+    hipLaunchKernelGGL((attn_dq_kernel<T, D, kDqWaves, decltype(heavy)::value>), dim3((unsigned)((size_t)nqt * H * B)),
+                       dim3(64 * kDqWaves), 0, stream, q, keys, values, o, dout, lse, dsum, dq, N, M, H, HKV, W, scale,
+                       scale_log2, nqt, order);
+  };
+  if (order != 0) dq_in(std::true_type{});
+  else dq_in(std::false_type{});
   auto dkv = [&](auto waves, int tiles) {
     hipLaunchKernelGGL((attn_dkv_kernel<T, D, decltype(waves)::value, kDkvWavesPerSimd, kDkvBlocks>),
                        dim3((unsigned)((size_t)tiles * HKV * B)), dim3(64 * decltype(waves)::value), 0, stream, q, keys,
